@@ -110,37 +110,48 @@ struct FastMath {
 // positive radicand in the range).
 //
 // The FP32 overloads do the same for binary32 (exponents within about +-90,
-// the solver's 1e-22..1e9 again): division is the reciprocal seed, one Newton
-// step and two remainder corrections of the IEEE sequence without v_div_scale
-// / v_div_fixup; square root takes the hardware estimate s (within 1 ulp) and
-// picks s - ulp, s or s + ulp from the signs of the exact residuals
-// x - (s -+ ulp) s, which decide on which side of the midpoints sqrt(x) lies.
+// the solver's 1e-22..1e9 again).  The reciprocal seed (v_rcp_f32, within 1 ulp)
+// after one Newton step is the correctly rounded reciprocal for every one of
+// the 2^23 mantissas, and one remainder correction of a r gives the correctly
+// rounded quotient for every one of the 2^46 pairs of mantissas (both checked
+// exhaustively on gfx950), so the second correction of the IEEE sequence is
+// left out.  The square root is x v_rsq_f32(x) with one residual correction,
+// correctly rounded for every x of the 2^24 in [1, 4) (exhaustive likewise),
+// in place of a choice among s - ulp, s and s + ulp by two residuals.  2 and 4
+// instructions fewer per quotient and root.
 struct RangedMath {
-  static __device__ __forceinline__ float div(float a, float b) {
-    const float nb = -b;
-    float r = __builtin_amdgcn_rcpf(b);
-    r = __builtin_fmaf(__builtin_fmaf(nb, r, 1.0f), r, r);
-    float q = a * r;
-    q = __builtin_fmaf(__builtin_fmaf(nb, q, a), r, q);
-    return __builtin_fmaf(__builtin_fmaf(nb, q, a), r, q);
+  static __device__ __forceinline__ float div(float a, float b) { return div_inv(a, b, recip(b)); }
+  static __device__ __forceinline__ float recip(float b) {
+    const float r = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+  }
+  // the start is not used: v_rcp_f32 and one step are as short
+  static __device__ __forceinline__ float recip_near(float b, float) { return recip(b); }
+  static __device__ __forceinline__ float div_inv(float a, float b, float r) {
+    const float q = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
   }
   static __device__ __forceinline__ float sqrt(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const int bits = __builtin_bit_cast(int, s);
-    const float dn = __builtin_bit_cast(float, bits - 1);
-    const float up = __builtin_bit_cast(float, bits + 1);
-    float t = __builtin_fmaf(-dn, s, x) <= 0.0f ? dn : s;
-    t = __builtin_fmaf(-up, s, x) > 0.0f ? up : t;
-    return t;
+    const float s = sqrt_pos(x);
+    return x == 0.0f ? x : s;
   }
-  static __device__ __forceinline__ float sqrt_pos(float x) { return sqrt(x); }
+  static __device__ __forceinline__ float sqrt_pos(float x) {
+    float y;
+    return sqrt_core(x, y);
+  }
+  // The reciprocal of the root s from v_rsq_f32's y instead of another
+  // v_rcp_f32: y with its last bit set and one Newton step against s.  For all
+  // x of the 2^24 in [1, 4) but 11 that is the correctly rounded 1/s, and the
+  // quotients of all 2^23 numerator mantissas by those 11 roots are correctly
+  // rounded too (both exhaustive; from y itself the step misses 1/s for
+  // s = 2 - 2^-23, where one quotient then rounds the other way).
   static __device__ __forceinline__ float sqrt_pos_inv(float x, float& inv) {
-    inv = 0.0f;
-    return sqrt(x);
+    float y;
+    const float s = sqrt_core(x, y);
+    y = __builtin_bit_cast(float, __builtin_bit_cast(int, y) | 1);
+    inv = __builtin_fmaf(y, __builtin_fmaf(-s, y, 1.0f), y);
+    return s;
   }
-  static __device__ __forceinline__ float div_inv(float a, float b, float) { return div(a, b); }
-  static __device__ __forceinline__ float recip(float) { return 0.0f; }
-  static __device__ __forceinline__ float recip_near(float, float) { return 0.0f; }
   // binary32: the same test as the double one below, evaluated in double,
   // where tol d is exact (48 bits), a - tol d is exact wherever it is near
   // h d (about 49 bits), and h d is exact and normal for every binary32 d
@@ -207,6 +218,11 @@ struct RangedMath {
   }
 
  private:
+  static __device__ __forceinline__ float sqrt_core(float x, float& y) {
+    y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+  }
   static __device__ __forceinline__ double sqrt_core(double x, double& hh) {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y;

@@ -186,3 +186,21 @@ def test_newton_stop_test_is_exact(gpu_lib, prec, dt):
     bad = np.nonzero(got != want)[0]
     assert 0.2 < want.mean() < 0.6
     assert bad.size == 0, f"{bad.size} of {a.size} decisions differ, first: {a[bad[:3]]} / {d[bad[:3]]}"
+
+
+def test_binary32_cores_over_every_mantissa(gpu_lib):
+    """FP32's reciprocal (one Newton step from the estimate) for each of the 2^23
+    mantissas, and its square root (one residual correction of x rsqrt(x)) for
+    each x in [1, 4): all correctly rounded.  A quotient by a root whose
+    reciprocal comes from the root's own estimate is checked for each x too."""
+    p = e2d.HydroParams(nx=8, ny=8, precision=e2d.PREC_FP32)
+    rng = np.random.default_rng(17)
+    for lo in (1.0, 2.0):
+        x = (np.float32(lo) * (1 + np.arange(1 << 23, dtype=np.float64) * 2.0 ** -23)).astype(np.float32)
+        got = e2d.pointwise(p, e2d.FN_SQRT, x.astype(np.float64))[:, 0].astype(np.float32)
+        assert np.array_equal(got, np.sqrt(x))
+        a = rng.uniform(1, 2, x.size).astype(np.float32)
+        got = e2d.pointwise(p, e2d.FN_DIV_ROOT, np.stack([a, x], axis=1).astype(np.float64)).astype(np.float32)
+        assert np.array_equal(got[:, 1], np.sqrt(x)) and np.array_equal(got[:, 0], a / np.sqrt(x))
+        got = e2d.pointwise(p, e2d.FN_DIV, np.stack([np.ones_like(x), x], axis=1).astype(np.float64))[:, 0]
+        assert np.array_equal(got.astype(np.float32), np.float32(1) / x)
