@@ -505,36 +505,27 @@ int e2d_run_steps(e2d_ctx* c, int nsteps, int* nStep) {
   }
   e2d::StepCfg cfg;
   cfg.dt_from_device = true;
-  if (c->p.implementation_version == E2D_IMPL_FUSED) {
-    // slot k holds the running invDt including the current input; the other
-    // slot must not exceed it before the first step writes there
-    if (int rc = fill_slot(c, 1 - k, 0.0)) return rc;
-    for (int s = 0; s < nsteps; ++s, ++n) {
-      cfg.buf_in = n % 2;
-      cfg.buf_out = 1 - cfg.buf_in;
-      cfg.slot_cur = k;
-      cfg.slot_next = 1 - k;
-      cfg.track_dt = true;
-      const e2d::TraceRange range("godunov_compute");
-      HIP_TRY(timed(c, E2D_TIMER_GODUNOV, [&] { return e2d::launch_fused_step(c->p, c->b, cfg, c->stream); }));
-      k = 1 - k;
-    }
-  } else {
-    // one slot: each step reads dt from slot k in its flux kernels, and its
-    // update kernel then folds the new state's CFL rates into slot k
-    for (int s = 0; s < nsteps; ++s, ++n) {
-      cfg.buf_in = n % 2;
-      cfg.buf_out = 1 - cfg.buf_in;
-      cfg.slot_cur = k;
-      cfg.track_dt = true;
-      const e2d::TraceRange range("godunov_compute");
+  // slot k holds the running invDt including the current input; the other
+  // slot must not exceed it before the first step writes there
+  if (int rc = fill_slot(c, 1 - k, 0.0)) return rc;
+  const bool fused = c->p.implementation_version == E2D_IMPL_FUSED;
+  for (int s = 0; s < nsteps; ++s, ++n) {
+    cfg.buf_in = n % 2;
+    cfg.buf_out = 1 - cfg.buf_in;
+    cfg.slot_cur = k;
+    cfg.slot_next = 1 - k;
+    cfg.track_dt = true;
+    const e2d::TraceRange range("godunov_compute");
+    if (!fused)
       HIP_TRY(timed(c, E2D_TIMER_BOUNDARIES,
                     [&] { return e2d::launch_boundaries(c->p, c->b, cfg.buf_in, c->stream); }));
-      HIP_TRY(timed(c, E2D_TIMER_GODUNOV,
-                    [&] { return e2d::launch_materialised_step(c->p, c->b, cfg, c->stream); }));
-    }
-    c->stages_valid = true;
+    HIP_TRY(timed(c, E2D_TIMER_GODUNOV, [&] {
+      return fused ? e2d::launch_fused_step(c->p, c->b, cfg, c->stream)
+                   : e2d::launch_materialised_step(c->p, c->b, cfg, c->stream);
+    }));
+    k = 1 - k;
   }
+  if (!fused) c->stages_valid = true;
   c->dev_slot = k;
   *nStep = n;
   return E2D_OK;

@@ -221,19 +221,8 @@ __device__ __forceinline__ void atomic_max_nonneg(double* dst, double v) {
   atomicMax(reinterpret_cast<unsigned long long*>(dst), static_cast<unsigned long long>(__double_as_longlong(v)));
 }
 
-// value of running-invDt slot `slot`: the maximum of its parts (uniform loads)
-__device__ __forceinline__ double invdt_read(const double* scal, int slot) {
-  const double* s = scal + slot * kInvdtSlot;
-  double m = s[0];
-#pragma unroll
-  for (int p = 1; p < kInvdtParts; ++p) {
-    const double x = s[p * kInvdtStride];
-    m = m > x ? m : x;
-  }
-  return m;
-}
-
-// The same for a whole wavefront (all 64 lanes active): lane l loads part
+// Value of running-invDt slot `slot`, the maximum of its parts, for a whole
+// wavefront (all 64 lanes active): lane l loads part
 // l mod kInvdtParts, one round trip for the slot, then a wave maximum; the
 // result is moved to scalar registers, where the uniform dt arithmetic stays.
 // In two halves, so that a kernel can issue the load early and reduce later:

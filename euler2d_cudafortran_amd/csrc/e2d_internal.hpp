@@ -12,9 +12,9 @@ namespace e2d {
 
 // Host-side trace range (roctx; rocprofv3 --marker-trace records it), named
 // after the reference's NVTX ranges (serial_ref/m_run.f90:195,264,336,387,502,571:
-// godunov_compute, compute_dt, convertToPrimitives, computeAndStoreFluxes,
-// updateHydro, make_boundaries).  It spans the enqueue of the kernels, which
-// the trace attributes to it.
+// godunov_compute, compute_dt, computeAndStoreFluxes, make_boundaries; the
+// conversion and the update have no kernels of their own).  It spans the
+// enqueue of the kernels, which the trace attributes to it.
 struct TraceRange {
   explicit TraceRange(const char* name) { roctxRangePushA(name); }
   ~TraceRange() { roctxRangePop(); }
@@ -54,8 +54,7 @@ struct StepCfg {
   bool dt_from_device = false;  // dt = cfl / (invDt slot slot_cur); else dt_host
   double dt_host = 0.0;
   int slot_cur = 0;
-  bool track_dt = false;  // fold the new state's CFL rate into invDt slot slot_next (fused
-                          // step) or slot_cur (materialised steps, after their flux kernels)
+  bool track_dt = false;  // fold the new state's CFL rate into invDt slot slot_next
   int slot_next = 1;
 };
 
@@ -63,7 +62,7 @@ size_t state_elem_bytes(int precision);   // storage type of the state
 size_t stage_elem_bytes(int precision, int stage);
 
 hipError_t launch_fused_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c, hipStream_t s);
-// prim .. update of the materialised version (boundaries launched separately)
+// the step of implementation versions 1 and 2, storing their stages (boundaries launched separately)
 hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c,
                                     hipStream_t s);
 hipError_t launch_boundaries(const e2d_params& p, const DevBuffers& b, int buf, hipStream_t s);

@@ -13,11 +13,11 @@
 // them.  The update epilogue also folds the CFL rate of the new state into the
 // running invDt of the next step (compute_dt, serial_ref/m_run.f90:248-312).
 //
-// Materialised step (implementationVersion 1): boundaries (launched by the
-// caller), primitive variables, slopes, face states, fluxes and update as
-// separate kernels with
-// every stage stored in HBM (cuf/m_HydroRun_gpu.cuf:393-418 structure, with
-// serial_ref arithmetic).
+// Materialised steps (implementationVersion 1: primitive variables, slopes,
+// face states and fluxes in HBM, cuf/m_HydroRun_gpu.cuf:393-418;
+// implementationVersion 2: primitive variables and fluxes, :421-446; both with
+// serial_ref arithmetic): boundaries (launched by the caller), then one kernel,
+// the fused step's march with every stage stored as it is formed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,12 +34,25 @@ namespace e2d {
 // ---------------------------------------------------------------------------
 // fused step
 
-constexpr int kStripOut = 60;  // output columns per wavefront
-// Independent wavefronts per workgroup of the fused and v2 flux kernels (their
+// Columns of a wavefront's strip: lane l of strip s holds column
+// s kOut + kFirst - kHalo + l, and the strip's own columns are those of the
+// lanes kHalo .. 63 - kHalo.  The fused step: 60 columns from the first
+// interior one, 2 halo columns each side.  With stages (STAGES != 0): 56
+// columns from column 0, so that every row that is stored begins and ends on a
+// 64-byte boundary.  With partial 64-byte pieces at every strip's edge, and
+// with stores that the caches keep, the stage arrays wrote at 3 TB/s; aligned
+// and non-temporal, at 5 (version 1 in FP64 at 2048^2, per step: 570 us,
+// aligned 530, both 385).
+template <int STAGES>
+struct Strip {
+  static constexpr int kHalo = STAGES ? 4 : 2, kOut = 64 - 2 * kHalo, kFirst = STAGES ? 0 : 2;
+};
+constexpr int kStripOut = Strip<0>::kOut;
+// Independent wavefronts per workgroup of the step kernels (their
 // wavefronts share nothing).  One per workgroup: measured on MI355X, the FP64
 // step takes 196.0-197.2 us at 2048^2 against 197.9-198.6 with four, and
 // 680.6-683.4 against 689.5-692.5 at 4096^2, with the same results; the float
-// kernels and the v2 flux kernel time the same either way, eight is slower.
+// kernels time the same either way, eight is slower.
 #ifndef E2D_WAVES_PER_BLOCK
 #define E2D_WAVES_PER_BLOCK 1
 #endif
@@ -80,7 +93,8 @@ struct StepArgs {
   int nshort, short_rows, short_base, nitems;
   int chunk;  // items per chunk dealt to one XCD (see fused_segment)
   int nstrips, tile;  // items are numbered over tiles of `tile` adjacent strips (see tile_item)
-  // Packed last strip: when the last strip has at most 12 (28) output columns,
+  // Packed last strip: when the last strip has at most 12 (28) output columns
+  // (8 or 24 with stages, whose halo is wider),
   // its wavefronts are split into groups of pk_w = 16 (32) lanes, each group on
   // its own segment of pk_rows rows, so the strip takes a quarter (half) of the
   // wavefronts.  Items [nlong - npk, nlong) are its wavefronts; segment k of the
@@ -89,6 +103,13 @@ struct StepArgs {
   // computes again with the same bits).  pk_w == 0: no packing; the last
   // strip's index is nstrips (the regular strips are 0 .. nstrips - 1).
   int pk_w, pk_rows, pk_nseg, npk;
+};
+
+// with the stage arrays of implementation versions 1 (all) and 2 (q, fx, fy)
+template <class P>
+struct StageArgs : StepArgs<P> {
+  typename P::T *q, *dqx, *dqy, *qxm, *qxp, *qym, *qyp;
+  typename P::U *fx, *fy;
 };
 
 // Item k of a tiled numbering of nstrips strips x nper segments each: tiles of
@@ -104,7 +125,7 @@ __device__ __forceinline__ void tile_item(int k, int nper, int nstrips, int tile
   strip = tc * tile + (in - seg * w);
 }
 
-// Segment (strip, rows [j0, j1)) of wavefront `wave` of block b; false for a
+// Segment (strip, rows [j0, j1), below ny + 2 + kMore) of wavefront `wave` of block b; false for a
 // wavefront without one.  Blocks go to the 8 XCDs round-robin (b % 8) and
 // start in order on each.  The long segments are dealt to the XCDs in chunks
 // of `chunk` consecutive items (vertical neighbours, which share rows, meet in
@@ -112,7 +133,7 @@ __device__ __forceinline__ void tile_item(int k, int nper, int nstrips, int tile
 // segments does not load one XCD), then the short ones the same way: every XCD
 // ends its share on short segments, which shortens the tail where the device
 // runs out of wavefronts.
-template <class P>
+template <int kMore, class P>
 __device__ __forceinline__ bool fused_segment(const StepArgs<P>& a, int b, int wave, int lane, int& strip, int& j0,
                                               int& j1, int& group_w) {
   int item;
@@ -129,8 +150,8 @@ __device__ __forceinline__ bool fused_segment(const StepArgs<P>& a, int b, int w
     seg = min((item - (a.nlong - a.npk)) * (64 / a.pk_w) + lane / a.pk_w, a.pk_nseg - 1);
     j0 = 2 + seg * a.pk_rows;
     j1 = j0 + a.pk_rows;
-    if (j1 > a.g.ny + 2) {
-      j1 = a.g.ny + 2;
+    if (j1 > a.g.ny + 2 + kMore) {
+      j1 = a.g.ny + 2 + kMore;
       j0 = j1 - a.pk_rows;
     }
     return true;
@@ -142,7 +163,7 @@ __device__ __forceinline__ bool fused_segment(const StepArgs<P>& a, int b, int w
   } else {
     tile_item(item, a.nshort, a.nstrips, a.tile, strip, seg);
     j0 = a.short_base + seg * a.short_rows;
-    j1 = min(j0 + a.short_rows, a.g.ny + 2);
+    j1 = min(j0 + a.short_rows, a.g.ny + 2 + kMore);
   }
   return true;
 }
@@ -197,10 +218,22 @@ __device__ __forceinline__ void prim_of(const Hydro<typename P::T>& h, const typ
   prim_of<P>(h, raw, q, irho);
 }
 
+// nothing in the step reads a stage array again: non-temporal
+template <class X>
+__device__ __forceinline__ void store_stage(X* a, const Grid& g, int i, int j, const X x[4]) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v) __builtin_nontemporal_store(x[v], a + at(g, i, j, v));
+}
+
 // kMinmod: instantiated for slope_type == 1 (the benchmark's minmod), whose
-// limiter then skips the products by st = 1 and the first-order select
-template <class P, int SOLVER, bool kMinmod>
-__device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
+// limiter then skips the products by st = 1 and the first-order select.
+// STAGES 1, 2: implementation versions 1 and 2, which store their stage arrays
+// on the way: q on every cell, slopes and face states on [1, size-2]^2, fx and
+// fy on [2, size-2]^2.  The input's ghost cells are filled, so every cell is
+// loaded as it is stored, and rows go one further than the update needs (the
+// reference's arrays hold the fluxes of row ny+2).
+template <class P, int SOLVER, bool kMinmod, int STAGES = 0, class Args>
+__device__ __forceinline__ void step_fused_body(const Args& a) {
   using T = typename P::T;
   using U = typename P::U;
   using S = typename P::S;
@@ -210,23 +243,30 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
   const int lane = threadIdx.x & 63;
   const Grid& g = a.g;
   int strip, j0, j1, group_w;
-  if (!fused_segment(a, blockIdx.x, wave, lane, strip, j0, j1, group_w)) return;  // whole wavefront: no barrier here
+  constexpr int kMore = STAGES != 0 ? 1 : 0;
+  if (!fused_segment<kMore, P>(a, blockIdx.x, wave, lane, strip, j0, j1, group_w)) return;  // whole wavefront: no barrier here
   // lanes per column group: 64, or 16 / 32 in the packed last strip, whose
   // groups march different rows (j0, j1 per lane, j1 - j0 the same for all)
   const int col = lane & (group_w - 1);
-  const int ci = strip * kStripOut + col;  // column of this lane
+  using SG = Strip<STAGES>;
+  const int ci = strip * SG::kOut + SG::kFirst - SG::kHalo + col;  // column of this lane
   const bool col_ok = ci < g.isize;
-  const int cl = col_ok ? ci : g.isize - 1;  // clamped column for loads
-  const bool out_lane = (col >= 2) && (col < group_w - 2) && (ci <= g.nx + 1);
+  const int cl = col_ok ? (STAGES != 0 ? max(ci, 0) : ci) : g.isize - 1;  // clamped column for loads
+  const bool own = col >= SG::kHalo && col < group_w - SG::kHalo;
+  const bool out_lane = own && ci <= g.nx + 1 && (STAGES == 0 || ci >= 2);
   // columns strip*60 .. strip*60+63 and rows j0-2 .. j1+1 all interior (never
   // in the packed strip, which holds the last columns)
 #if E2D_FUSED_PLAIN
-  const bool plain = __builtin_amdgcn_readfirstlane(group_w == 64 && strip * kStripOut >= 2 &&
+  const bool plain = STAGES != 0 || __builtin_amdgcn_readfirstlane(group_w == 64 && strip * kStripOut >= 2 &&
                                                     strip * kStripOut + 63 <= g.nx + 1 && j0 - 2 >= 2 &&
                                                     j1 + 1 <= g.ny + 1 ? 1 : 0) != 0;
 #else
-  const bool plain = false;
+  const bool plain = STAGES != 0;
 #endif
+  // with stages: the columns whose q, slopes and face states, and fluxes this lane stores
+  const bool q_lane = own && ci < g.isize;
+  const bool slope_lane = own && ci >= 1 && ci <= g.nx + 2;
+  const bool flux_lane = own && ci >= 2 && ci <= g.nx + 2;
   // iterations r = j0 - 1 .. j1 of the row loop, the same number on every lane
   const int n_it = __builtin_amdgcn_readfirstlane(j1 - j0 + 2);
 
@@ -247,6 +287,12 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
   prim_of<P>(h, raw, qa);
   source_cell<P>(a, cl, col_ok, j0 - 1, plain, raw_b);
   prim_of<P>(h, raw_b, qb, irb);
+  if constexpr (STAGES != 0) {
+    if (j0 == 2 && q_lane) {
+      store_stage(a.q, g, ci, 0, qa);
+      store_stage(a.q, g, ci, 1, qb);
+    }
+  }
 
   // dt of this step (serial_ref/m_run.f90:308, 384-385)
   U dt;
@@ -287,7 +333,10 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) raw[v] = raw_next[v];
     if (it < n_it - 1) {  // r + 2 <= j1 + 1
-      if (plain) {
+      if constexpr (STAGES != 0) {
+        // clamped to the last row there is, past which the results are not used
+        fetch_cell<P>(a, cl, min(r + 2, g.jsize - 1), true, raw_next);
+      } else if (plain) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) raw_next[v] = in_row[v * g.plane];
       } else {
@@ -309,6 +358,10 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
     for (int v = 0; v < 4; ++v) rows_in[(slot_w * 4 + v) * 64 + lane] = raw[v];
 #endif
     prim_of<P>(h, raw, qc, irc);
+    if constexpr (STAGES != 0) {
+      // row r+1 in [j0, j1), and the topmost row with the last segment
+      if (q_lane && (it < n_it - 2 || (it == n_it - 2 && j1 == g.ny + 2 + kMore))) store_stage(a.q, g, ci, r + 1, qc);
+    }
 
     // slopes and trace sources of row r
     T qxm[4], qxp[4], dqx[4], dqy[4], s[4];
@@ -319,6 +372,21 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
     }
     cell_slopes<kMinmod>(h, qb, qxp, qxm, qc, qa, dqx, dqy);
     trace_sources<T, M>(h, qb, dqx, dqy, s, irb);
+    if constexpr (STAGES == 1) {
+      if (slope_lane && ((it >= 1 && it < n_it - 1) || (it == 0 && j0 == 2))) {
+        store_stage(a.dqx, g, ci, r, dqx);
+        store_stage(a.dqy, g, ci, r, dqy);
+        T f[4];
+        face_state(h, qb, dqx, s, dtdx, true, f);
+        store_stage(a.qxm, g, ci, r, f);
+        face_state(h, qb, dqx, s, dtdx, false, f);
+        store_stage(a.qxp, g, ci, r, f);
+        face_state(h, qb, dqy, s, dtdy, true, f);
+        store_stage(a.qym, g, ci, r, f);
+        face_state(h, qb, dqy, s, dtdy, false, f);
+        store_stage(a.qyp, g, ci, r, f);
+      }
+    }
 
     // y-face between rows r-1 and r
     if (it >= 1) {  // r >= j0
@@ -327,6 +395,9 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
       riemann_y<T, M, SOLVER>(h, ymax_prev, ymin, f);
 #pragma unroll
       for (int v = 0; v < 4; ++v) fy_cur[v] = static_cast<U>(f[v]) * dtdyU;
+      if constexpr (STAGES != 0) {
+        if (it < n_it - 1 && flux_lane) store_stage(a.fy, g, ci, r, fy_cur);
+      }
     }
     face_state(h, qb, dqy, s, dtdy, true, ymax_prev);
 
@@ -340,6 +411,9 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
       riemann<T, M, SOLVER>(h, xl, xmin, gd, f);
 #pragma unroll
       for (int v = 0; v < 4; ++v) fx_cur[v] = static_cast<U>(f[v]) * dtdxU;
+      if constexpr (STAGES != 0) {
+        if (flux_lane) store_stage(a.fx, g, ci, r, fx_cur);
+      }
     }
 
     // conservative update of row r-1 (updateHydro, serial_ref/m_run.f90:504-513)
@@ -347,7 +421,7 @@ __device__ __forceinline__ void step_fused_body(const StepArgs<P>& a) {
       U fxr[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) fxr[v] = from_right(fx_prev[v]);
-      if (out_lane) {
+      if (out_lane && (STAGES == 0 || r - 1 <= g.ny + 1)) {
         const int jr = r - 1;
 #if E2D_FUSED_UOLD_LDS
         const int slot_r = slot_w == 2 ? 0 : slot_w + 1;  // slot of row r - 1
@@ -419,13 +493,30 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) __attribute__((amdgpu_waves_pe
   step_fused_body<P, 2, false>(a);
 }
 
+// The materialised versions' step (STAGES 1 and 2) on the same march.  As six
+// and four kernels that passed q, slopes, face states and fluxes through HBM,
+// version 1 moved 3.5 GB and version 2 1.4 GB per 2048^2 FP64 step, at the rate
+// of a copy; here each stage is written once and read by nothing (1.67 GB and
+// 0.8 GB): 740 -> 340 us and 356 -> 220 us per step.  Version 1 is bound by its
+// writes; in FP64 it is held at 2 wavefronts per SIMD, since at 3 it spills
+// 60 B per lane (385 us).  Version 2 is bound by VALU issue, as the fused step.
+template <class P, int STAGES>
+constexpr int staged_waves() {
+  return STAGES == 1 && sizeof(typename P::T) == 8 ? 2 : fused_waves<P>();
+}
+template <class P, int SOLVER, bool kMinmod, int STAGES>
+__global__ __launch_bounds__(64 * kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(staged_waves<P, STAGES>())))
+void k_step_staged(const StageArgs<P> a) {
+  step_fused_body<P, SOLVER, kMinmod, STAGES>(a);
+}
+
 static int env_int(const char* name, int dflt) {
   const char* v = getenv(name);
   return v && *v ? atoi(v) : dflt;
 }
 
 // Rows per long segment where the whole-round plan does not apply (small
-// grids; the v2 flux kernel).  Each segment re-primes its rolling rows (two
+// grids).  Each segment re-primes its rolling rows (two
 // extra row loads and primitive conversions, one extra row of y-faces), so
 // long segments are cheaper per row; short ones give more wavefronts to hide
 // latency and balance the data-dependent Newton work, and on small grids a
@@ -464,7 +555,7 @@ static int waves_per_simd(const void* kernel) {
   return std::max(1, blocks_per_cu * kWavesPerBlock / 4);
 }
 
-// Segment plan of a fused launch over nstrips strips.  Long segments cover
+// Segment plan of a fused launch over ncols columns and ny rows.  Long segments cover
 // about 80% (FP64) or 88% (FP32, mixed) of each strip's rows, in as many
 // segments per strip as fill k whole rounds of the device's resident
 // wavefronts (k the least that keeps them within 40 rows); short ones of a
@@ -481,12 +572,14 @@ static int waves_per_simd(const void* kernel) {
 // E2D_FUSED_SEG_ROWS or E2D_FUSED_LONG_PCT select that plan with the given
 // values, E2D_FUSED_SHORT_ROWS the short length; the environment is read at
 // every launch.  Returns the number of blocks.
-template <class P>
-static int plan_segments(StepArgs<P>& a, int nstrips_all, int ny, int wps, int resident) {
+template <class SG, class P>
+static int plan_segments(StepArgs<P>& a, int ncols, int ny, int wps, int resident) {
+  const int nstrips_all = (ncols + SG::kOut - 1) / SG::kOut;
   // the packed last strip (see StepArgs): output columns left for it
-  const int last_cols = a.g.nx - kStripOut * (nstrips_all - 1);
+  const int last_cols = ncols - SG::kOut * (nstrips_all - 1);
   int pk_w = 0;
-  if (nstrips_all >= 2 && env_int("E2D_FUSED_PACK", 1) != 0) pk_w = last_cols <= 12 ? 16 : (last_cols <= 28 ? 32 : 0);
+  if (nstrips_all >= 2 && env_int("E2D_FUSED_PACK", 1) != 0)
+    pk_w = last_cols <= 16 - 2 * SG::kHalo ? 16 : (last_cols <= 32 - 2 * SG::kHalo ? 32 : 0);
   const int nstrips = pk_w ? nstrips_all - 1 : nstrips_all;
   const int groups = pk_w ? 64 / pk_w : 1;  // segments per packed wavefront
   int R = 0, L = 0;
@@ -543,27 +636,30 @@ static int plan_segments(StepArgs<P>& a, int nstrips_all, int ny, int wps, int r
   return dealt_blocks(a.nlong, a.nitems, a.chunk, kWavesPerBlock);
 }
 
-template <class P, int SOLVER, bool kMinmod>
-static hipError_t launch_fused(StepArgs<P>& a, int nstrips, hipStream_t st) {
-  const void* kernel;
-  if constexpr (SOLVER == 2)
-    kernel = reinterpret_cast<const void*>(k_step_fused_hllc<P>);
+template <class P, int SOLVER, bool kMinmod, int STAGES = 0, class Args>
+static hipError_t launch_fused(Args& a, hipStream_t st) {
+  void (*kernel)(const Args);
+  if constexpr (STAGES != 0)
+    kernel = k_step_staged<P, SOLVER, kMinmod, STAGES>;
+  else if constexpr (SOLVER == 2)
+    kernel = k_step_fused_hllc<P>;
   else
-    kernel = reinterpret_cast<const void*>(k_step_fused<P, SOLVER, kMinmod>);
-  thread_local const int wps = waves_per_simd(kernel);
-  const int nblocks = plan_segments(a, nstrips, a.g.ny, wps, 4 * wps * device_cus());
-  if constexpr (SOLVER == 2)
-    hipLaunchKernelGGL((k_step_fused_hllc<P>), dim3(nblocks), dim3(64 * kWavesPerBlock), 0, st, a);
-  else
-    hipLaunchKernelGGL((k_step_fused<P, SOLVER, kMinmod>), dim3(nblocks), dim3(64 * kWavesPerBlock), 0, st, a);
+    kernel = k_step_fused<P, SOLVER, kMinmod>;
+  thread_local const int wps = waves_per_simd(reinterpret_cast<const void*>(kernel));
+  // with stages: every column, and the fluxes of row ny+2
+  const int nblocks = plan_segments<Strip<STAGES>, P>(a, STAGES != 0 ? a.g.isize : a.g.nx,
+                                                   STAGES != 0 ? a.g.ny + 1 : a.g.ny, wps, 4 * wps * device_cus());
+  hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(64 * kWavesPerBlock), 0, st, a);
   return hipGetLastError();
 }
 
-template <class P>
+template <class P, int STAGES>
 static hipError_t fused_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c, hipStream_t st) {
-  StepArgs<P> a;
-  a.hT = make_hydro<typename P::T>(p);
-  a.hU = make_hydro<typename P::U>(p);
+  using T = typename P::T;
+  using U = typename P::U;
+  std::conditional_t<STAGES != 0, StageArgs<P>, StepArgs<P>> a{};
+  a.hT = make_hydro<T>(p);
+  a.hU = make_hydro<U>(p);
   a.g = make_grid(p, b);
   a.uin = static_cast<typename P::S*>(b.u[c.buf_in]);
   a.uout = static_cast<typename P::S*>(b.u[c.buf_out]);
@@ -573,16 +669,33 @@ static hipError_t fused_step(const e2d_params& p, const DevBuffers& b, const Ste
   a.track_dt = c.track_dt ? 1 : 0;
   a.slot_next = c.slot_next;
   a.dt_host = c.dt_host;
+  if constexpr (STAGES != 0) {
+    a.q = static_cast<T*>(b.stage[E2D_STAGE_Q]);
+    a.fx = static_cast<U*>(b.stage[E2D_STAGE_FX]);
+    a.fy = static_cast<U*>(b.stage[E2D_STAGE_FY]);
+    a.dqx = static_cast<T*>(b.stage[E2D_STAGE_DQX]);
+    a.dqy = static_cast<T*>(b.stage[E2D_STAGE_DQY]);
+    a.qxm = static_cast<T*>(b.stage[E2D_STAGE_QXM]);
+    a.qxp = static_cast<T*>(b.stage[E2D_STAGE_QXP]);
+    a.qym = static_cast<T*>(b.stage[E2D_STAGE_QYM]);
+    a.qyp = static_cast<T*>(b.stage[E2D_STAGE_QYP]);
+  }
   const bool hllc = p.riemann_solver == E2D_RIEMANN_HLLC;
-  const bool minmod = !hllc && p.slope_type == 1;
-  const int nstrips = (p.nx + kStripOut - 1) / kStripOut;
-  if (hllc) return launch_fused<P, 2, false>(a, nstrips, st);
-  if (minmod) return launch_fused<P, 0, true>(a, nstrips, st);
-  return launch_fused<P, 0, false>(a, nstrips, st);
+  if (hllc) return launch_fused<P, 2, false, STAGES>(a, st);
+  if (p.slope_type == 1) return launch_fused<P, 0, true, STAGES>(a, st);
+  return launch_fused<P, 0, false, STAGES>(a, st);
 }
 
 hipError_t launch_fused_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c, hipStream_t s) {
-  return with_precision(p.precision, [&](auto pol) { return fused_step<decltype(pol)>(p, b, c, s); });
+  return with_precision(p.precision, [&](auto pol) { return fused_step<decltype(pol), 0>(p, b, c, s); });
+}
+
+hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c, hipStream_t s) {
+  const TraceRange range("computeAndStoreFluxes");
+  return with_precision(p.precision, [&](auto pol) {
+    using P = decltype(pol);
+    return p.implementation_version == E2D_IMPL_FLUX_STORE ? fused_step<P, 2>(p, b, c, s) : fused_step<P, 1>(p, b, c, s);
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -625,7 +738,7 @@ hipError_t launch_tangent_step(const e2d_params& p, const DevBuffers& b, int buf
   const dim3 grid((g.isize + 63) / 64, (g.jsize + 3) / 4);
   hipLaunchKernelGGL(k_pack_dual, grid, dim3(256), 0, st, g, static_cast<const double*>(b.u[buf]), v_in,
                      static_cast<Dual*>(dual_in));
-  StepArgs<PDual> a;
+  StepArgs<PDual> a{};
   a.hT = make_hydro<Dual>(p);
   a.hU = a.hT;
   a.g = g;
@@ -637,7 +750,7 @@ hipError_t launch_tangent_step(const e2d_params& p, const DevBuffers& b, int buf
   a.track_dt = 0;
   a.slot_next = 1;
   a.dt_host = dt;
-  if (hipError_t e = launch_fused<PDual, 0, false>(a, (p.nx + kStripOut - 1) / kStripOut, st)) return e;
+  if (hipError_t e = launch_fused<PDual, 0, false>(a, st)) return e;
   hipLaunchKernelGGL(k_unpack_dual, grid, dim3(256), 0, st, g, static_cast<const Dual*>(dual_out), v_out);
   return hipGetLastError();
 }
@@ -780,334 +893,6 @@ hipError_t launch_words_differ(const void* a, const void* b, size_t bytes, doubl
                      dim3(256), 0, s, static_cast<const unsigned long long*>(a),
                      static_cast<const unsigned long long*>(b), n, flag);
   return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// materialised steps (implementationVersion 1: q, slopes, face states and
-// fluxes in HBM; implementationVersion 2: q and fluxes in HBM)
-
-template <class P>
-struct MatArgs {
-  Hydro<typename P::T> hT;
-  Hydro<typename P::U> hU;
-  Grid g;
-  const typename P::S* uin;
-  typename P::S* uout;
-  typename P::T *q, *dqx, *dqy, *qxm, *qxp, *qym, *qyp;
-  typename P::U *fx, *fy;
-  double* scal;
-  int dt_from_device, slot_cur;
-  double dt_host;
-  int nsegs, seg_rows, seg_groups;  // k_flux_store row segments
-  int track_dt;  // k_update folds the new state's CFL rates into invDt slot slot_cur
-};
-
-// kWave: called with all 64 lanes of the wavefront active (wave-parallel read)
-template <bool kWave = false, class P>
-__device__ __forceinline__ void step_dt(const MatArgs<P>& a, typename P::U& dtdx, typename P::U& dtdy) {
-  using U = typename P::U;
-  U dt = static_cast<U>(a.dt_host);
-  if (a.dt_from_device)
-    dt = a.hU.cfl / static_cast<U>(kWave ? invdt_read_wave(a.scal, a.slot_cur) : invdt_read(a.scal, a.slot_cur));
-  dtdx = dt / a.hU.dx;
-  dtdy = dt / a.hU.dy;
-}
-
-// convertToPrimitives over all cells (serial_ref/m_run.f90:338-354)
-template <class P>
-__global__ __launch_bounds__(256) void k_prim(const MatArgs<P> a) {
-  using T = typename P::T;
-  const int i = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
-  if (i >= a.g.isize || j >= a.g.jsize) return;
-  T u[4], q[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) u[v] = static_cast<T>(a.uin[at(a.g, i, j, v)]);
-  cons_to_prim<T, typename P::M>(a.hT, u, q);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) a.q[at(a.g, i, j, v)] = q[v];
-}
-
-// slopes of cells [1, size-2]^2
-template <class P>
-__global__ __launch_bounds__(256) void k_slopes(const MatArgs<P> a) {
-  using T = typename P::T;
-  const int i = 1 + blockIdx.x * 64 + (threadIdx.x & 63);
-  const int j = 1 + blockIdx.y * 4 + (threadIdx.x >> 6);
-  if (i > a.g.isize - 2 || j > a.g.jsize - 2) return;
-  T q[4], xp[4], xm[4], yp[4], ym[4], dx[4], dy[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    q[v] = a.q[at(a.g, i, j, v)];
-    xp[v] = a.q[at(a.g, i + 1, j, v)];
-    xm[v] = a.q[at(a.g, i - 1, j, v)];
-    yp[v] = a.q[at(a.g, i, j + 1, v)];
-    ym[v] = a.q[at(a.g, i, j - 1, v)];
-  }
-  cell_slopes(a.hT, q, xp, xm, yp, ym, dx, dy);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    a.dqx[at(a.g, i, j, v)] = dx[v];
-    a.dqy[at(a.g, i, j, v)] = dy[v];
-  }
-}
-
-// the four face states of cells [1, size-2]^2
-template <class P>
-__global__ __launch_bounds__(256) void k_trace(const MatArgs<P> a) {
-  using T = typename P::T;
-  using U = typename P::U;
-  const int i = 1 + blockIdx.x * 64 + (threadIdx.x & 63);
-  const int j = 1 + blockIdx.y * 4 + (threadIdx.x >> 6);
-  if (i > a.g.isize - 2 || j > a.g.jsize - 2) return;
-  U dtdxU, dtdyU;
-  step_dt(a, dtdxU, dtdyU);
-  const T dtdx = static_cast<T>(dtdxU), dtdy = static_cast<T>(dtdyU);
-  T q[4], dx[4], dy[4], s[4], f[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    q[v] = a.q[at(a.g, i, j, v)];
-    dx[v] = a.dqx[at(a.g, i, j, v)];
-    dy[v] = a.dqy[at(a.g, i, j, v)];
-  }
-  trace_sources<T, typename P::M>(a.hT, q, dx, dy, s);
-  face_state(a.hT, q, dx, s, dtdx, true, f);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) a.qxm[at(a.g, i, j, v)] = f[v];
-  face_state(a.hT, q, dx, s, dtdx, false, f);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) a.qxp[at(a.g, i, j, v)] = f[v];
-  face_state(a.hT, q, dy, s, dtdy, true, f);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) a.qym[at(a.g, i, j, v)] = f[v];
-  face_state(a.hT, q, dy, s, dtdy, false, f);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) a.qyp[at(a.g, i, j, v)] = f[v];
-}
-
-// fluxes of the faces of computeAndStoreFluxes, (i, j) in [2, size-2]^2
-// (serial_ref/m_run.f90:389-480)
-template <class P, int SOLVER>
-__global__ __launch_bounds__(256) void k_flux(const MatArgs<P> a) {
-  using T = typename P::T;
-  using U = typename P::U;
-  const int i = 2 + blockIdx.x * 64 + (threadIdx.x & 63);
-  const int j = 2 + blockIdx.y * 4 + (threadIdx.x >> 6);
-  if (i > a.g.isize - 2 || j > a.g.jsize - 2) return;
-  U dtdx, dtdy;
-  step_dt(a, dtdx, dtdy);
-  T l[4], r[4], gd[4], f[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    l[v] = a.qxm[at(a.g, i - 1, j, v)];
-    r[v] = a.qxp[at(a.g, i, j, v)];
-  }
-  riemann<T, typename P::M, SOLVER>(a.hT, l, r, gd, f);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) a.fx[at(a.g, i, j, v)] = static_cast<U>(f[v]) * dtdx;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    l[v] = a.qym[at(a.g, i, j - 1, v)];
-    r[v] = a.qyp[at(a.g, i, j, v)];
-  }
-  riemann_y<T, typename P::M, SOLVER>(a.hT, l, r, f);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) a.fy[at(a.g, i, j, v)] = static_cast<U>(f[v]) * dtdy;
-}
-
-// computeFluxesAndStore (implementationVersion 2, cuf/m_HydroRun_gpu.cuf:747-884,
-// with serial_ref's arithmetic): fx(i, j) (face between i-1 and i) and fy(i, j)
-// (face between j-1 and j) for (i, j) in [2, isize-2]^2, times dt/dx and dt/dy,
-// from the primitives k_prim stored.  The reference computes slopes and traces
-// three times per cell (own, i-1, j-1); here, as in the fused step, a wavefront
-// owns a strip of 64 columns (60 stored, lanes 2..61) and marches up a segment
-// of rows, forming each cell's slopes, trace sources and face states once: the
-// left state of an x-face comes from lane-1, the lower state of a y-face from
-// the previous row, in registers.  Same bits as the per-cell formulation.
-template <class P, int SOLVER, bool kMinmod = false>
-__global__ __launch_bounds__(64 * kWavesPerBlock) void k_flux_store(const MatArgs<P> a) {
-  using T = typename P::T;
-  using U = typename P::U;
-  using M = typename P::M;
-  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  int strip, group;
-  strip_and_group<false>(lb, a.seg_groups, strip, group);
-  const int seg = group * kWavesPerBlock + wave;
-  if (seg >= a.nsegs) return;  // whole wavefront leaves: no barrier in this kernel
-
-  const Grid& g = a.g;
-  const int ci = strip * kStripOut + lane;  // column of this lane
-  const int cl = ci < g.isize ? ci : g.isize - 1;
-  const bool out_lane = lane >= 2 && lane < 62 && ci <= g.isize - 2;
-  const int j0 = 2 + seg * a.seg_rows;
-  const int j1 = min(j0 + a.seg_rows, g.jsize - 1);  // stored rows [j0, j1)
-  U dtdxU, dtdyU;
-  step_dt<true>(a, dtdxU, dtdyU);
-  const T dtdx = static_cast<T>(dtdxU), dtdy = static_cast<T>(dtdyU);
-  const Hydro<T>& h = a.hT;
-
-  T qa[4], qb[4], qc[4], ymax_prev[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    qa[v] = a.q[at(g, cl, j0 - 2, v)];
-    qb[v] = a.q[at(g, cl, j0 - 1, v)];
-  }
-  for (int r = j0 - 1; r < j1; ++r) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) qc[v] = a.q[at(g, cl, r + 1, v)];
-    T qxm[4], qxp[4], dqx[4], dqy[4], s[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      qxm[v] = from_left(qb[v]);
-      qxp[v] = from_right(qb[v]);
-    }
-    cell_slopes<kMinmod>(h, qb, qxp, qxm, qc, qa, dqx, dqy);
-    trace_sources<T, M>(h, qb, dqx, dqy, s);
-    if (r >= j0) {
-      // y-face between rows r-1 and r
-      T ymin[4], f[4];
-      face_state(h, qb, dqy, s, dtdy, false, ymin);
-      riemann_y<T, M, SOLVER>(h, ymax_prev, ymin, f);
-      if (out_lane) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) a.fy[at(g, ci, r, v)] = static_cast<U>(f[v]) * dtdyU;
-      }
-      // x-face between columns ci-1 and ci
-      T xmin[4], xmax[4], xl[4], gd[4];
-      face_state(h, qb, dqx, s, dtdx, false, xmin);
-      face_state(h, qb, dqx, s, dtdx, true, xmax);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) xl[v] = from_left(xmax[v]);
-      riemann<T, M, SOLVER>(h, xl, xmin, gd, f);
-      if (out_lane) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) a.fx[at(g, ci, r, v)] = static_cast<U>(f[v]) * dtdxU;
-      }
-    }
-    face_state(h, qb, dqy, s, dtdy, true, ymax_prev);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      qa[v] = qb[v];
-      qb[v] = qc[v];
-    }
-  }
-}
-
-// updateHydro over the interior (serial_ref/m_run.f90:504-513).  With
-// track_dt, the CFL rate of each new cell in the compute_dt window [2, n]
-// (0-based) is folded into the running invDt (compute_dt of the new state,
-// serial_ref/m_run.f90:248-312): a wave maximum, a block maximum through LDS,
-// one atomic maximum per block.  This step's dt was read from that slot by the
-// flux kernels, which have completed; the maximum is order-independent.
-template <class P>
-__global__ __launch_bounds__(256) void k_update(const MatArgs<P> a) {
-  using U = typename P::U;
-  using S = typename P::S;
-  __shared__ double red[4];
-  const int i = 2 + blockIdx.x * 64 + (threadIdx.x & 63);
-  const int j = 2 + blockIdx.y * 4 + (threadIdx.x >> 6);
-  const bool cell = i <= a.g.nx + 1 && j <= a.g.ny + 1;
-  U rate = U(0);
-  if (cell) {
-    U un[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      U flux_tot = a.fx[at(a.g, i, j, v)] - a.fx[at(a.g, i + 1, j, v)];
-      flux_tot = a.fy[at(a.g, i, j, v)] - a.fy[at(a.g, i, j + 1, v)] + flux_tot;
-      const S sn = static_cast<S>(static_cast<U>(a.uin[at(a.g, i, j, v)]) + flux_tot);
-      a.uout[at(a.g, i, j, v)] = sn;
-      un[v] = static_cast<U>(sn);
-    }
-    if (a.track_dt && i <= a.g.nx && j <= a.g.ny) rate = cfl_rate<U, typename P::MU>(a.hU, un);
-  }
-  if (!a.track_dt) return;  // uniform: the whole block leaves before the barrier
-  const double m = wave_max(static_cast<double>(rate));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double x = red[0];
-    for (int k = 1; k < 4; ++k) x = x > red[k] ? x : red[k];
-    invdt_fold(a.scal, a.slot_cur, static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x), x);
-  }
-}
-
-template <class P>
-static hipError_t materialised_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c,
-                                    hipStream_t st) {
-  using T = typename P::T;
-  using U = typename P::U;
-  MatArgs<P> a;
-  a.hT = make_hydro<T>(p);
-  a.hU = make_hydro<U>(p);
-  a.g = make_grid(p, b);
-  a.uin = static_cast<const typename P::S*>(b.u[c.buf_in]);
-  a.uout = static_cast<typename P::S*>(b.u[c.buf_out]);
-  a.q = static_cast<T*>(b.stage[E2D_STAGE_Q]);
-  a.fx = static_cast<U*>(b.stage[E2D_STAGE_FX]);
-  a.fy = static_cast<U*>(b.stage[E2D_STAGE_FY]);
-  a.dqx = static_cast<T*>(b.stage[E2D_STAGE_DQX]);
-  a.dqy = static_cast<T*>(b.stage[E2D_STAGE_DQY]);
-  a.qxm = static_cast<T*>(b.stage[E2D_STAGE_QXM]);
-  a.qxp = static_cast<T*>(b.stage[E2D_STAGE_QXP]);
-  a.qym = static_cast<T*>(b.stage[E2D_STAGE_QYM]);
-  a.qyp = static_cast<T*>(b.stage[E2D_STAGE_QYP]);
-  a.scal = b.scal;
-  a.dt_from_device = c.dt_from_device ? 1 : 0;
-  a.slot_cur = c.slot_cur;
-  a.dt_host = c.dt_host;
-  a.track_dt = c.track_dt ? 1 : 0;
-  const int S_ = p.nx + 4, J_ = p.ny + 4;
-  const dim3 fgrid((S_ - 3 + 63) / 64, (J_ - 3 + 3) / 4);
-  {
-    const TraceRange range("convertToPrimitives");
-    hipLaunchKernelGGL(k_prim<P>, dim3((S_ + 63) / 64, (J_ + 3) / 4), dim3(256), 0, st, a);
-  }
-  {
-    const TraceRange range("computeAndStoreFluxes");
-    if (p.implementation_version == E2D_IMPL_FLUX_STORE) {
-      // stored rows and columns [2, size-2]; segment length as for the fused step
-      const bool hllc = p.riemann_solver == E2D_RIEMANN_HLLC;
-      const bool minmod = !hllc && p.slope_type == 1;
-      const void* kernel = hllc ? reinterpret_cast<const void*>(k_flux_store<P, 2>)
-                                : (minmod ? reinterpret_cast<const void*>(k_flux_store<P, 0, true>)
-                                          : reinterpret_cast<const void*>(k_flux_store<P, 0>));
-      thread_local const void* cached_kernel = nullptr;
-      thread_local int cached_wps = 3;
-      if (kernel != cached_kernel) {
-        cached_wps = waves_per_simd(kernel);
-        cached_kernel = kernel;
-      }
-      a.seg_rows = fused_seg_rows(p.ny, cached_wps);
-      a.nsegs = (J_ - 3 + a.seg_rows - 1) / a.seg_rows;
-      a.seg_groups = (a.nsegs + kWavesPerBlock - 1) / kWavesPerBlock;
-      const dim3 mgrid(((S_ - 3 + kStripOut - 1) / kStripOut) * a.seg_groups);
-      if (hllc)
-        hipLaunchKernelGGL((k_flux_store<P, 2>), mgrid, dim3(64 * kWavesPerBlock), 0, st, a);
-      else if (minmod)
-        hipLaunchKernelGGL((k_flux_store<P, 0, true>), mgrid, dim3(64 * kWavesPerBlock), 0, st, a);
-      else
-        hipLaunchKernelGGL((k_flux_store<P, 0>), mgrid, dim3(64 * kWavesPerBlock), 0, st, a);
-    } else {
-      hipLaunchKernelGGL(k_slopes<P>, dim3((S_ - 2 + 63) / 64, (J_ - 2 + 3) / 4), dim3(256), 0, st, a);
-      hipLaunchKernelGGL(k_trace<P>, dim3((S_ - 2 + 63) / 64, (J_ - 2 + 3) / 4), dim3(256), 0, st, a);
-      if (p.riemann_solver == E2D_RIEMANN_HLLC)
-        hipLaunchKernelGGL((k_flux<P, 2>), fgrid, dim3(256), 0, st, a);
-      else
-        hipLaunchKernelGGL((k_flux<P, 0>), fgrid, dim3(256), 0, st, a);
-    }
-  }
-  {
-    const TraceRange range("updateHydro");
-    hipLaunchKernelGGL(k_update<P>, dim3((p.nx + 63) / 64, (p.ny + 3) / 4), dim3(256), 0, st, a);
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c,
-                                    hipStream_t s) {
-  return with_precision(p.precision, [&](auto pol) { return materialised_step<decltype(pol)>(p, b, c, s); });
 }
 
 // ---------------------------------------------------------------------------

@@ -339,3 +339,59 @@ def test_float_variants_against_fp64(gpu_lib, prec):
     errs = [rel_l1(a[i, i, v], b[i, i, v]) for v in range(4)]
     print(f"precision {prec} vs fp64, 256^2 diagonal problem, 200 steps: rel L1 {['%.3e' % e for e in errs]}")
     assert all(e <= bnd for e, bnd in zip(errs, FLOAT_VARIANT_BOUNDS[prec])), errs
+
+
+# ---------------------------------------------------------------------------
+# stage arrays at strip, segment and grid edges
+
+# 60 and 120 columns leave the flux column nx+2 a strip of its own; 59 and 119
+# fill the last strip with it; 130 x 151 has a packed last strip
+@pytest.mark.parametrize("nx, ny", [(4, 4), (60, 16), (119, 33), (120, 9), (130, 151)])
+@pytest.mark.parametrize("impl, prec, st", [(1, e2d.PREC_FP64, 1), (1, e2d.PREC_FP32, 2), (1, e2d.PREC_MIXED, 1),
+                                            (2, e2d.PREC_FP64, 2), (2, e2d.PREC_FP32_NATIVE, 1)])
+def test_stage_arrays_are_the_routines_values(gpu_lib, nx, ny, impl, prec, st):
+    """Every stage array of a step against the device routines (e2d_pointwise, pinned to the
+    reference's by their own tests) applied to the stages before it, bit for bit, on every
+    cell the reference's arrays hold; cells outside stay zero."""
+    p = _params(nx, ny, impl, prec, slope_type=st, boundary_type_xmax=2, boundary_type_ymin=3, boundary_type_ymax=3)
+    T = np.float64 if prec == e2d.PREC_FP64 else np.float32
+    U = np.float32 if prec == e2d.PREC_FP32 else np.float64
+    rng = np.random.default_rng(nx)
+    u = np.empty((nx + 4, ny + 4, 4))
+    u[..., 0] = rng.uniform(0.2, 2, u.shape[:2])
+    u[..., 2:] = rng.uniform(-0.5, 0.5, u.shape[:2] + (2,))
+    u[..., 1] = rng.uniform(0.5, 3, u.shape[:2]) + 0.5 * (u[..., 2:] ** 2).sum(-1) / u[..., 0]
+    with e2d.HydroRun(p) as run:
+        run.upload(0, u)
+        dt = run.compute_dt(0)
+        run.godunov_unsplit(0, dt)
+        names = ("q", "dqx", "dqy", "qxm", "qxp", "qym", "qyp", "fx", "fy") if impl == 1 else ("q", "fx", "fy")
+        a = {n: run.download_stage(n) for n in names}
+        u0 = run.download(0)  # ghost cells filled
+    dtdx, dtdy = (float(U(dt) / (U(1) / U(n))) for n in (nx, ny))
+
+    def at(func, *cols):
+        x = np.concatenate([np.broadcast_to(c, cols[0].shape[:2] + (np.shape(c)[-1],)) for c in cols], axis=-1)
+        return e2d.pointwise(p, func, x.reshape(-1, x.shape[-1])).reshape(x.shape[:2] + (-1,))
+
+    q = at(e2d.FN_PRIM, u0)[..., :4]
+    assert _same(a["q"], q)
+    c, xp, xm, yp, ym = q[1:-1, 1:-1], q[2:, 1:-1], q[:-2, 1:-1], q[1:-1, 2:], q[1:-1, :-2]
+    dq = at(e2d.FN_SLOPE, c, xp, xm, yp, ym)
+    dx, dy = dq[..., :4], dq[..., 4:]
+    ratios = np.array([T(dtdx), T(dtdy)], dtype=np.float64)
+    face = {}
+    for n, k in (("qxm", 1), ("qxp", 0), ("qym", 3), ("qyp", 2)):
+        face[n] = at(e2d.FN_TRACE, c, dx, dy, ratios, np.array([float(k)]))
+    if impl == 1:
+        for n, want in (("dqx", dx), ("dqy", dy), *face.items()):
+            full = np.zeros_like(q)
+            full[1:-1, 1:-1] = want
+            assert _same(a[n], full), (n, _diff_report(a[n], full))
+    sw = [0, 1, 3, 2]  # velocities exchanged for a y-face
+    fx = at(e2d.FN_RIEMANN, face["qxm"][:-1, 1:], face["qxp"][1:, 1:])[..., 4:]
+    fy = at(e2d.FN_RIEMANN, face["qym"][1:, :-1][..., sw], face["qyp"][1:, 1:][..., sw])[..., 4:][..., sw]
+    for n, f, r in (("fx", fx, dtdx), ("fy", fy, dtdy)):
+        full = np.zeros_like(q)
+        full[2:-1, 2:-1] = (f.astype(U) * U(r)).astype(np.float64)
+        assert _same(a[n], full), (n, _diff_report(a[n], full))
