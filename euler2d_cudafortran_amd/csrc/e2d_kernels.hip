@@ -493,6 +493,165 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) __attribute__((amdgpu_waves_pe
   step_fused_body<P, 2, false>(a);
 }
 
+// ---------------------------------------------------------------------------
+// The fused step on tiles, for grids too small to fill the device with marching
+// wavefronts (there a step lasts as long as one wavefront's chain of row
+// iterations).  A workgroup takes a strip of 64 columns (60 stored) and R rows,
+// one row a wavefront and R + 2 wavefronts, and its rows meet in LDS: each
+// wavefront forms its row's primitives (the outer two also those of the rows
+// beyond), then its slopes, face states and x-face problems, then the y-face
+// problems below its row, with the row below's upper face states from LDS, then
+// its update, with the y-flux above from LDS.  The chain is one row with two
+// Riemann problems whatever R is.  It forms the marching kernel's values by the
+// same routines on the same operands, so the bits are the same.
+// Each wavefront holds one row only: 80 VGPRs in FP64 (6 wavefronts per SIMD,
+// against the march's 3) and about 50 in the float variants.  us per FP64 step,
+// march against tiles: 128^2 11.1, 8.1; 250 x 130 11.3, 8.4; 512^2 21.4, 20.2;
+// 768^2 44.8, 37.3.  On grids that fill the device (2048^2: 178 against 225)
+// the barriers and the rows formed twice cost more than the chain saves.
+constexpr int kTileMaxRows = 14;
+template <class P>
+constexpr int tile_waves() {
+  return sizeof(typename P::T) == 8 ? 6 : 8;
+}
+// rows of LDS (4 variables x 64 lanes of T) of a tile of R rows: primitives and
+// the lower states, then fluxes, of the y-faces
+constexpr int tile_lds_rows(int rows) { return (rows + 4) + (rows + 1); }
+
+template <class P, bool kMinmod>
+__global__ __launch_bounds__(64 * (kTileMaxRows + 2)) __attribute__((amdgpu_waves_per_eu(tile_waves<P>())))
+void k_step_tile(const StepArgs<P> a) {
+  using T = typename P::T;
+  using U = typename P::U;
+  using S = typename P::S;
+  using M = typename P::M;
+  extern __shared__ __align__(16) unsigned char tile_mem[];
+  const Grid& g = a.g;
+  const Hydro<T>& h = a.hT;
+  const int R = a.seg_rows;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = static_cast<int>(threadIdx.x & 63);
+  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
+  const int strip = lb / a.nsegs;
+  const int j0 = 2 + (lb - strip * a.nsegs) * R;
+  const int nr = min(R, g.ny + 2 - j0);  // this tile's rows [j0, j0 + nr)
+  const int ci = strip * kStripOut + lane;
+  const bool col_ok = ci < g.isize;
+  const int cl = col_ok ? ci : g.isize - 1;
+  const bool out_lane = lane >= 2 && lane < 62 && ci <= g.nx + 1;
+  const int left = lane > 0 ? lane - 1 : 0, right = lane < 63 ? lane + 1 : 63;
+  const int r = j0 - 1 + wave;  // the wavefront's row
+  const bool has_row = wave < nr + 2, x_row = wave >= 1 && wave <= nr, y_face = wave >= 1 && wave <= nr + 1;
+  const bool up_row = wave <= nr;
+  const bool plain = strip * kStripOut >= 2 && strip * kStripOut + 63 <= g.nx + 1 && j0 >= 4 && j0 + nr <= g.ny;
+
+  T* const q_lds = reinterpret_cast<T*>(tile_mem);  // row k: grid row j0 - 2 + k
+  T* const y_lds = q_lds + (R + 4) * 256;           // y-face k, between rows j0-1+k and j0+k
+
+  double invdt_cur = 0.0;
+  if (a.dt_from_device) invdt_cur = invdt_part(a.scal, a.slot_cur);
+  T q[4], irho;
+  if (has_row) {
+    S raw[4], raw2[4];
+    const bool ends = wave == 0 || wave == nr + 1;
+    const int r2 = wave == 0 ? r - 1 : r + 1;
+    fetch_cell<P>(a, cl, r, plain, raw);
+    if (ends) fetch_cell<P>(a, cl, r2, plain, raw2);
+    source_cell<P>(a, cl, col_ok, r, plain, raw);
+    prim_of<P>(h, raw, q, irho);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) q_lds[((wave + 1) * 4 + v) * 64 + lane] = q[v];
+    if (ends) {
+      T q2[4];
+      source_cell<P>(a, cl, col_ok, r2, plain, raw2);
+      prim_of<P>(h, raw2, q2);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) q_lds[((r2 - j0 + 2) * 4 + v) * 64 + lane] = q2[v];
+    }
+  }
+  U dt;
+  if (a.dt_from_device) {
+    invdt_cur = invdt_reduce(invdt_cur);
+    dt = a.hU.cfl / static_cast<U>(invdt_cur);
+  } else {
+    dt = static_cast<U>(a.dt_host);
+  }
+  const U dtdxU = dt / a.hU.dx;
+  const U dtdyU = dt / a.hU.dy;
+  const T dtdx = static_cast<T>(dtdxU);
+  const T dtdy = static_cast<T>(dtdyU);
+  __syncthreads();
+
+  T ymin[4], fx[4] = {T(0), T(0), T(0), T(0)};
+  S uold[4] = {S(0), S(0), S(0), S(0)};
+  if (has_row) {
+    T dqx[4], dqy[4], s[4];
+    {
+      const T* const qr = q_lds + (wave + 1) * 256;
+      T xm[4], xp[4], ym[4], yp[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        xm[v] = qr[v * 64 + left];
+        xp[v] = qr[v * 64 + right];
+        ym[v] = qr[v * 64 + lane - 256];
+        yp[v] = qr[v * 64 + lane + 256];
+      }
+      cell_slopes<kMinmod>(h, q, xp, xm, yp, ym, dqx, dqy);
+    }
+    trace_sources<T, M>(h, q, dqx, dqy, s, irho);
+    if (up_row) {
+      T f[4];
+      face_state(h, q, dqy, s, dtdy, true, f);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) y_lds[(wave * 4 + v) * 64 + lane] = f[v];
+    }
+    face_state(h, q, dqy, s, dtdy, false, ymin);
+    if (x_row) {
+      T xl[4], xr[4], gd[4];
+      face_state(h, q, dqx, s, dtdx, true, xl);
+      face_state(h, q, dqx, s, dtdx, false, xr);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) xl[v] = from_left(xl[v]);
+      riemann<T, M, 0>(h, xl, xr, gd, fx);
+    }
+  }
+  __syncthreads();
+  T* const fy = y_lds + (wave - 1) * 256;  // y-face below the wavefront's row
+  T fyl[4];
+  if (y_face) {
+    T lo[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) lo[v] = fy[v * 64 + lane];
+    if (x_row && out_lane) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) uold[v] = a.uin[at(g, ci, r, v)];
+    }
+    riemann_y<T, M, 0>(h, lo, ymin, fyl);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) fy[v * 64 + lane] = fyl[v];
+  }
+  __syncthreads();
+  if (x_row) {
+    U rate_max = U(0), un[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const U fxs = static_cast<U>(fx[v]) * dtdxU;
+      const U flux_tot = (static_cast<U>(fyl[v]) * dtdyU - static_cast<U>(fy[v * 64 + lane + 256]) * dtdyU) +
+                         (fxs - from_right(fxs));
+      const S sn = static_cast<S>(static_cast<U>(uold[v]) + flux_tot);
+      if (out_lane) a.uout[at(g, ci, r, v)] = sn;
+      un[v] = static_cast<U>(sn);
+    }
+    if (a.track_dt) {
+      if (out_lane && ci <= g.nx && r <= g.ny) rate_max = cfl_rate<U, typename P::MU>(a.hU, un);
+      double m = static_cast<double>(rate_max);
+      m = m > invdt_cur ? m : invdt_cur;  // running maximum carries over
+      m = wave_max(m);
+      if (lane == 0) invdt_fold(a.scal, a.slot_next, static_cast<int>(blockIdx.x) * R + wave, m);
+    }
+  }
+}
+
 // The materialised versions' step (STAGES 1 and 2) on the same march.  As six
 // and four kernels that passed q, slopes, face states and fluxes through HBM,
 // version 1 moved 3.5 GB and version 2 1.4 GB per 2048^2 FP64 step, at the rate
@@ -636,8 +795,56 @@ static int plan_segments(StepArgs<P>& a, int ncols, int ny, int wps, int residen
   return dealt_blocks(a.nlong, a.nitems, a.chunk, kWavesPerBlock);
 }
 
+// Rows per tile, or 0 for the marching kernel.  Tiles up to 2,700 cells per
+// compute unit in FP64 and 2,400 in the float variants (about 830^2 and 780^2),
+// where the two cross.  us per step, march against tiles: 640^2 FP64 36.6,
+// 30.5; 800^2 48.1, 45.7; 900^2 53.7, 57.4; 1000 x 610 FP32 27.2, 23.5; 800^2
+// 27.6, 29.7; 640^2 fp32_native 20.8, 16.5; 800^2 23.6, 26.4.  A step on tiles
+// takes about as long as the wavefronts on the busiest compute unit, ceil(tiles
+// / compute units) (R + 2), and longer by the root of the residency lost where
+// they come in several rounds of tiles of R + 2 wavefronts that do not fill it
+// (512^2 FP64: 10 rows 20.2, 6 rows 23.7; 900^2: 6 rows 50.2, 14 rows 53.1).
+// The rows with the least of that are taken, among equals the fewest.
+// E2D_TILE_ROWS gives the rows (0: march), and any E2D_FUSED_* plan selects the
+// march it describes.
+static int plan_tile_rows(const Grid& g, int waves_per_cu, int most_cells) {
+  const int forced = env_int("E2D_TILE_ROWS", -1);
+  if (forced >= 0) return std::min(forced, kTileMaxRows);
+  const int cus = device_cus();
+  if (static_cast<int64_t>(g.nx) * g.ny > static_cast<int64_t>(most_cells) * cus) return 0;
+  for (const char* name : {"E2D_FUSED_SEG_ROWS", "E2D_FUSED_SHORT_ROWS", "E2D_FUSED_LONG_PCT", "E2D_FUSED_COVER_PCT",
+                           "E2D_FUSED_CHUNK", "E2D_FUSED_TILE", "E2D_FUSED_PACK"})
+    if (getenv(name)) return 0;
+  const int64_t strips = (g.nx + kStripOut - 1) / kStripOut;
+  int best = 0;
+  double least = 0.0;
+  for (int rows = 1; rows <= kTileMaxRows; ++rows) {
+    const int64_t tiles = strips * ((g.ny + rows - 1) / rows);
+    const int64_t per_cu = (tiles + cus - 1) / cus;
+    const int resident = std::max(1, waves_per_cu / (rows + 2));
+    double cost = static_cast<double>(per_cu * (rows + 2)) * (per_cu * (rows + 2));
+    if (per_cu > resident) cost *= static_cast<double>(waves_per_cu) / (resident * (rows + 2));
+    if (best == 0 || cost < least) {
+      best = rows;
+      least = cost;
+    }
+  }
+  return best;
+}
+
 template <class P, int SOLVER, bool kMinmod, int STAGES = 0, class Args>
 static hipError_t launch_fused(Args& a, hipStream_t st) {
+  if constexpr (SOLVER == 0 && STAGES == 0 && sizeof(typename P::T) <= 8) {
+    const int rows = plan_tile_rows(a.g, 4 * tile_waves<P>(), sizeof(typename P::T) == 8 ? 2700 : 2400);
+    if (rows > 0) {
+      a.seg_rows = rows;
+      a.nsegs = (a.g.ny + rows - 1) / rows;
+      const int nstrips = (a.g.nx + kStripOut - 1) / kStripOut;
+      hipLaunchKernelGGL((k_step_tile<P, kMinmod>), dim3(nstrips * a.nsegs), dim3(64 * (rows + 2)),
+                         tile_lds_rows(rows) * 256 * sizeof(typename P::T), st, a);
+      return hipGetLastError();
+    }
+  }
   void (*kernel)(const Args);
   if constexpr (STAGES != 0)
     kernel = k_step_staged<P, SOLVER, kMinmod, STAGES>;

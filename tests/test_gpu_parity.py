@@ -395,3 +395,27 @@ def test_stage_arrays_are_the_routines_values(gpu_lib, nx, ny, impl, prec, st):
         full = np.zeros_like(q)
         full[2:-1, 2:-1] = (f.astype(U) * U(r)).astype(np.float64)
         assert _same(a[n], full), (n, _diff_report(a[n], full))
+
+
+# the tile kernel: a single strip, 1 and 20 columns left for the last strip, rows that do not
+# divide into tiles, tiles higher than the grid, every number of rows' extremes
+@pytest.mark.parametrize("rows", [1, 2, 5, 14])
+@pytest.mark.parametrize("nx, ny, bc, st", [(4, 4, (1, 1, 1, 1), 1), (61, 17, (1, 2, 3, 1), 2), (80, 43, (3, 3, 2, 1), 0),
+                                            (60, 29, (2, 1, 3, 3), 1)])
+def test_tile_rows_vs_march(gpu_lib, monkeypatch, nx, ny, bc, st, rows):
+    """The fused step on tiles equals the marching kernel (which the plan tests pin to the
+    oracle) bit for bit in every precision: both buffers, ghost cells and corners included,
+    and the running invDt, after a host-driven step and 9 device-resident ones."""
+    for prec in (e2d.PREC_FP64, e2d.PREC_FP32, e2d.PREC_FP32_NATIVE, e2d.PREC_MIXED):
+        got = []
+        for tile in (0, rows):
+            monkeypatch.setenv("E2D_TILE_ROWS", str(tile))
+            kw = dict(zip(("boundary_type_xmin", "boundary_type_xmax", "boundary_type_ymin", "boundary_type_ymax"), bc))
+            with e2d.HydroRun(_params(nx, ny, 0, prec, slope_type=st, **kw)) as run:
+                run.init("diag")
+                run.godunov_unsplit(0, run.compute_dt(0))
+                run.nStep = 1
+                run.run_steps(9)
+                got.append((run.download(0), run.download(1), run.invdt))
+        (a0, a1, ai), (b0, b1, bi) = got
+        assert _same(b0, a0) and _same(b1, a1) and ai == bi, (prec, _diff_report(b0, a0))
