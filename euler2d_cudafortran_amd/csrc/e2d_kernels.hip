@@ -726,8 +726,9 @@ static int waves_per_simd(const void* kernel) {
 // (which leaves 9% of the long segments for a second round); FP32 12 rows
 // 134-136 against 139-140; fp32_native 106.3 against 107.1; 4096^2 FP64 37 rows
 // (two rounds) 711 against 716, 74 rows (one round) 719.  Where the rounds
-// would give segments of fewer than 8 rows (grids up to about 1024^2) the
-// plan is long segments of fused_seg_rows rows over 75% of the rows.
+// would give segments of fewer than 8 rows (grids up to about 1200^2) the
+// plan is segments of one length in FP64 (below), and long segments of
+// fused_seg_rows rows over 75% of the rows otherwise.
 // E2D_FUSED_SEG_ROWS or E2D_FUSED_LONG_PCT select that plan with the given
 // values, E2D_FUSED_SHORT_ROWS the short length; the environment is read at
 // every launch.  Returns the number of blocks.
@@ -769,6 +770,22 @@ static int plan_segments(StepArgs<P>& a, int ncols, int ny, int wps, int residen
       const int pk = ((ny + R - 1) / R + groups - 1) / groups;
       if (pk == npk) break;
       npk = pk;
+    }
+  }
+  // FP64 grids of about 800^2 to 1400^2: segments of one length, the least that
+  // lets all of them start at once.  us per step against long segments over 75%
+  // of the rows: 850^2 44.1 against 52.8, 1024^2 57.7 against 66.4, 1200^2 73.3
+  // against 82.7, 1400^2 93.4 against 93.9 (the float variants gain and lose 2%).
+  if (R == 0 && !forced && sizeof(typename P::T) == 8) {
+    int rows = 1;
+    auto wavefronts = [&](int r) {
+      const int segs = (ny + r - 1) / r;
+      return nstrips * static_cast<int64_t>(segs) + (pk_w ? (segs + groups - 1) / groups : 0);
+    };
+    while (rows < 40 && wavefronts(rows) > resident) ++rows;
+    if (rows >= 4 && wavefronts(rows) <= resident) {
+      R = rows;
+      L = (ny + R - 1) / R;
     }
   }
   if (R == 0) {
