@@ -94,7 +94,9 @@ struct e2d_ctx {
   int device = 0;
   int isize = 0, jsize = 0;
   double* staging = nullptr;  // float64 host-layout staging array on the device
-  double* d_sums = nullptr;
+  // pinned host memory that kernels write small results to (block maxima of
+  // compute_dt, the sums) and slots are copied to: no staging copy behind them
+  double* pinned = nullptr;
   // running invDt of compute_dt: authoritative on the host when dev_slot < 0,
   // else in device slot dev_slot of b.scal (the maximum of its parts)
   double invdt = 0.0;
@@ -141,6 +143,8 @@ int check_buf(int buf) {
   return E2D_OK;
 }
 
+constexpr int kPinnedDoubles = std::max(e2d::kMaxInvdtBlocks, e2d::kInvdtSlot);
+
 size_t host_elems(const e2d_ctx* c) { return static_cast<size_t>(c->isize) * c->jsize * 4; }
 
 // set every part of running-invDt slot `slot` to v
@@ -151,9 +155,9 @@ int fill_slot(e2d_ctx* c, int slot, double v) {
 
 // value of running-invDt slot `slot` (the maximum of its parts); synchronous
 int read_slot(e2d_ctx* c, int slot, double* v) {
-  double parts[e2d::kInvdtSlot];
-  HIP_TRY(hipMemcpyAsync(parts, c->b.scal + slot * e2d::kInvdtSlot, sizeof(parts), hipMemcpyDeviceToHost,
-                         c->stream));
+  const double* parts = c->pinned;
+  HIP_TRY(hipMemcpyAsync(c->pinned, c->b.scal + slot * e2d::kInvdtSlot, e2d::kInvdtSlot * sizeof(double),
+                         hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   double m = parts[0];
   for (int p = 1; p < e2d::kInvdtParts; ++p) m = m > parts[p * e2d::kInvdtStride] ? m : parts[p * e2d::kInvdtStride];
@@ -254,7 +258,7 @@ void free_all(e2d_ctx* c) {
   if (c->b.scal) (void)hipFree(c->b.scal), c->b.scal = nullptr;
   if (c->b.partial) (void)hipFree(c->b.partial), c->b.partial = nullptr;
   if (c->staging) (void)hipFree(c->staging), c->staging = nullptr;
-  if (c->d_sums) (void)hipFree(c->d_sums), c->d_sums = nullptr;
+  if (c->pinned) (void)hipHostFree(c->pinned), c->pinned = nullptr;
   if (c->stream) (void)hipStreamDestroy(c->stream), c->stream = nullptr;
 }
 
@@ -351,7 +355,7 @@ int e2d_create(const e2d_params* p, e2d_ctx** out) {
             hipMalloc(reinterpret_cast<void**>(&c->b.scal), e2d::kScalDoubles * sizeof(double)) ==
                 hipSuccess &&
             hipMalloc(reinterpret_cast<void**>(&c->b.partial), e2d::kSumBlocks * 4 * sizeof(double)) == hipSuccess &&
-            hipMalloc(reinterpret_cast<void**>(&c->d_sums), 4 * sizeof(double)) == hipSuccess;
+            hipHostMalloc(reinterpret_cast<void**>(&c->pinned), kPinnedDoubles * sizeof(double)) == hipSuccess;
   if (ok && p->implementation_version != E2D_IMPL_FUSED) {
     // version 1 keeps every stage; version 2 only q, fx and fy (cuf/m_HydroRun_gpu.cuf:93-105)
     const int nstages = p->implementation_version == E2D_IMPL_MATERIALISED ? e2d::kNumStages : E2D_STAGE_FY + 1;
@@ -453,9 +457,20 @@ int e2d_compute_dt(e2d_ctx* c, int useU, double* dt) {
   if (!dt) return fail(E2D_ERR_ARG, "dt is NULL");
   if (int rc = pull_invdt(c)) return rc;
   const int buf = (useU == 0) ? 0 : 1;
-  if (int rc = fill_slot(c, 2, c->invdt)) return rc;
-  HIP_TRY(timed(c, E2D_TIMER_DT, [&] { return e2d::launch_max_invdt(c->p, c->b, buf, 2, c->stream); }));
-  if (int rc = read_slot(c, 2, &c->invdt)) return rc;
+  // each block writes its maximum to host memory; their maximum by bit pattern
+  // is that of the device's atomic maxima (non-negative values)
+  int nblocks = 0;
+  HIP_TRY(timed(c, E2D_TIMER_DT,
+                [&] { return e2d::launch_block_invdt(c->p, c->b, buf, c->pinned, &nblocks, c->stream); }));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  uint64_t most = 0;
+  std::memcpy(&most, &c->invdt, sizeof(most));
+  for (int k = 0; k < nblocks; ++k) {
+    uint64_t bits;
+    std::memcpy(&bits, c->pinned + k, sizeof(bits));
+    most = std::max(most, bits);
+  }
+  std::memcpy(&c->invdt, &most, sizeof(most));
   *dt = dt_of(c->p, c->invdt);
   return E2D_OK;
 }
@@ -500,14 +515,15 @@ int e2d_run_steps(e2d_ctx* c, int nsteps, int* nStep) {
   if (k < 0) {
     // compute_dt of the current input, folded into the running maximum
     k = 0;
-    if (int rc = fill_slot(c, k, c->invdt)) return rc;
+    HIP_TRY(e2d::launch_start_slots(c->b.scal, nullptr, c->invdt, c->stream));
     HIP_TRY(timed(c, E2D_TIMER_DT, [&] { return e2d::launch_max_invdt(c->p, c->b, n % 2, k, c->stream); }));
+  } else if (int rc = fill_slot(c, 1 - k, 0.0)) {
+    return rc;
   }
+  // slot k holds the running invDt including the current input; the other slot
+  // does not exceed it before the first step writes there
   e2d::StepCfg cfg;
   cfg.dt_from_device = true;
-  // slot k holds the running invDt including the current input; the other
-  // slot must not exceed it before the first step writes there
-  if (int rc = fill_slot(c, 1 - k, 0.0)) return rc;
   const bool fused = c->p.implementation_version == E2D_IMPL_FUSED;
   for (int s = 0; s < nsteps; ++s, ++n) {
     cfg.buf_in = n % 2;
@@ -560,9 +576,9 @@ int e2d_sums(e2d_ctx* c, int buf, double out[4]) {
   if (int rc = check_ctx(c)) return rc;
   if (int rc = check_buf(buf)) return rc;
   if (!out) return fail(E2D_ERR_ARG, "out is NULL");
-  HIP_TRY(e2d::launch_sums(c->p, c->b, buf, c->d_sums, c->stream));
-  HIP_TRY(hipMemcpyAsync(out, c->d_sums, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(e2d::launch_sums(c->p, c->b, buf, c->pinned, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
+  std::copy_n(c->pinned, 4, out);
   return E2D_OK;
 }
 
@@ -948,8 +964,7 @@ int e2d_run_steps_noalloc(const e2d_params* p, void* d_u, void* d_u2, int64_t pi
   b.scal = scr;
   // slot 0: the running invDt folded with the current input's CFL rate
   // (compute_dt); slot 1: zero until the first step folds into it
-  HIP_TRY(e2d::launch_fill_from(scr, e2d::kInvdtSlot, d_invdt, st));
-  HIP_TRY(e2d::launch_fill(scr + e2d::kInvdtSlot, e2d::kInvdtSlot, 0.0, st));
+  HIP_TRY(e2d::launch_start_slots(scr, d_invdt, 0.0, st));
   HIP_TRY(e2d::launch_max_invdt(*p, b, nStep % 2, 0, st));
   e2d::StepCfg cfg;
   cfg.dt_from_device = true;

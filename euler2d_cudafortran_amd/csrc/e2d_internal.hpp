@@ -28,11 +28,11 @@ constexpr int kNumStages = 9;  // E2D_STAGE_Q .. E2D_STAGE_QYP
 // per 128-byte line, and its value is their maximum: the atomic maxima that
 // every wavefront of a step folds in spread over independent lines instead of
 // serialising on one address (at 2048^2 a step folds 6,000 of them).  Slots 0
-// and 1 ping-pong between steps; slot 2 serves compute_dt.
+// and 1 ping-pong between steps.
 constexpr int kInvdtParts = 32;
 constexpr int kInvdtStride = 16;                          // doubles between parts
 constexpr int kInvdtSlot = kInvdtParts * kInvdtStride;    // doubles per slot
-constexpr int kInvdtSlots = 3;
+constexpr int kInvdtSlots = 2;
 constexpr int kScalDoubles = kInvdtSlots * kInvdtSlot;  // doubles in the allocation
 
 // Device memory of one run.  State element (i, j, v), 0-based, of buffer b
@@ -47,6 +47,7 @@ struct DevBuffers {
 };
 
 constexpr int kSumBlocks = 240;
+constexpr int kMaxInvdtBlocks = 2048;
 
 // How a step obtains dt.
 struct StepCfg {
@@ -68,9 +69,15 @@ hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, co
 hipError_t launch_boundaries(const e2d_params& p, const DevBuffers& b, int buf, hipStream_t s);
 // atomic max of the CFL rate over the compute_dt window of buffer buf into invDt slot `slot`
 hipError_t launch_max_invdt(const e2d_params& p, const DevBuffers& b, int buf, int slot, hipStream_t s);
+// the same maximum as one value per block, out[0 .. *nblocks) (at most
+// kMaxInvdtBlocks), for a caller that takes their maximum: out may be host
+// memory that the device writes
+hipError_t launch_block_invdt(const e2d_params& p, const DevBuffers& b, int buf, double* out, int* nblocks,
+                              hipStream_t s);
 hipError_t launch_fill(double* dst, int n, double v, hipStream_t s);
-// dst[0..n) = *src (src a device address)
-hipError_t launch_fill_from(double* dst, int n, const double* src, hipStream_t s);
+// running-invDt slots 0 and 1 of scal: every part of slot 0 becomes *src (a
+// device address), or v where src is null, and of slot 1 zero
+hipError_t launch_start_slots(double* scal, const double* src, double v, hipStream_t s);
 // *dst = value of the running-invDt slot starting at `slot` (the maximum of its parts)
 hipError_t launch_slot_value(const double* slot, double* dst, hipStream_t s);
 // *flag (device) = 1 when the two device arrays of `bytes` bytes differ in any bit, else 0
@@ -78,7 +85,8 @@ hipError_t launch_words_differ(const void* a, const void* b, size_t bytes, doubl
 hipError_t launch_init_problem(const e2d_params& p, const DevBuffers& b, int problem,
                                const double* bumps /* 16 x 5 host values */, hipStream_t s);
 hipError_t launch_zero_state(const e2d_params& p, const DevBuffers& b, int buf, hipStream_t s);
-hipError_t launch_sums(const e2d_params& p, const DevBuffers& b, int buf, double* d_out4, hipStream_t s);
+// out4: device memory, or host memory that the device writes
+hipError_t launch_sums(const e2d_params& p, const DevBuffers& b, int buf, double* out4, hipStream_t s);
 // conversion between the float64 host layout (isize*jsize*4, Fortran order)
 // and the pitched device state, through a device staging array of doubles
 hipError_t launch_pack(const e2d_params& p, const DevBuffers& b, int buf, const double* d_src, hipStream_t s);

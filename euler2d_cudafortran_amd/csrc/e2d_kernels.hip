@@ -1028,7 +1028,8 @@ hipError_t launch_boundaries(const e2d_params& p, const DevBuffers& b, int buf, 
 
 template <class P>
 __global__ __launch_bounds__(256) void k_max_invdt(const Hydro<typename P::U> h, const Grid g,
-                                                    const typename P::S* __restrict__ u, double* scal, int slot) {
+                                                    const typename P::S* __restrict__ u, double* scal, int slot,
+                                                    double* per_block) {
   using U = typename P::U;
   __shared__ double red[4];
   const int w = g.nx - 1, hgt = g.ny - 1;  // window extent
@@ -1050,24 +1051,36 @@ __global__ __launch_bounds__(256) void k_max_invdt(const Hydro<typename P::U> h,
   if (threadIdx.x == 0) {
     double x = red[0];
     for (int k = 1; k < 4; ++k) x = x > red[k] ? x : red[k];
-    invdt_fold(scal, slot, blockIdx.x, x);
+    if (per_block)
+      per_block[blockIdx.x] = x;
+    else
+      invdt_fold(scal, slot, blockIdx.x, x);
   }
 }
 
 template <class P>
-static hipError_t max_invdt(const e2d_params& p, const DevBuffers& b, int buf, int slot, hipStream_t st) {
+static hipError_t max_invdt(const e2d_params& p, const DevBuffers& b, int buf, int slot, double* per_block,
+                            int* nblocks, hipStream_t st) {
   const Grid g = make_grid(p, b);
   const int64_t n = static_cast<int64_t>(p.nx - 1) * (p.ny - 1);
   int nb = static_cast<int>((n + 255) / 256);
-  if (nb > 2048) nb = 2048;
+  if (nb > kMaxInvdtBlocks) nb = kMaxInvdtBlocks;
   if (nb < 1) nb = 1;
   hipLaunchKernelGGL(k_max_invdt<P>, dim3(nb), dim3(256), 0, st, make_hydro<typename P::U>(p), g,
-                     static_cast<const typename P::S*>(b.u[buf]), b.scal, slot);
+                     static_cast<const typename P::S*>(b.u[buf]), b.scal, slot, per_block);
+  if (nblocks) *nblocks = nb;
   return hipGetLastError();
 }
 
 hipError_t launch_max_invdt(const e2d_params& p, const DevBuffers& b, int buf, int slot, hipStream_t s) {
-  return with_precision(p.precision, [&](auto pol) { return max_invdt<decltype(pol)>(p, b, buf, slot, s); });
+  return with_precision(p.precision,
+                        [&](auto pol) { return max_invdt<decltype(pol)>(p, b, buf, slot, nullptr, nullptr, s); });
+}
+
+hipError_t launch_block_invdt(const e2d_params& p, const DevBuffers& b, int buf, double* out, int* nblocks,
+                              hipStream_t s) {
+  return with_precision(p.precision,
+                        [&](auto pol) { return max_invdt<decltype(pol)>(p, b, buf, 0, out, nblocks, s); });
 }
 
 __global__ void k_fill(double* dst, int n, double v) {
@@ -1080,13 +1093,14 @@ hipError_t launch_fill(double* dst, int n, double v, hipStream_t s) {
   return hipGetLastError();
 }
 
-__global__ void k_fill_from(double* dst, int n, const double* src) {
+__global__ void k_start_slots(double* scal, const double* src, double v) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) dst[t] = *src;
+  if (t < kInvdtSlot) scal[t] = src ? *src : v;
+  else if (t < 2 * kInvdtSlot) scal[t] = 0.0;
 }
 
-hipError_t launch_fill_from(double* dst, int n, const double* src, hipStream_t s) {
-  hipLaunchKernelGGL(k_fill_from, dim3((n + 63) / 64), dim3(64), 0, s, dst, n, src);
+hipError_t launch_start_slots(double* scal, const double* src, double v, hipStream_t s) {
+  hipLaunchKernelGGL(k_start_slots, dim3(2 * kInvdtSlot / 256), dim3(256), 0, s, scal, src, v);
   return hipGetLastError();
 }
 
@@ -1221,16 +1235,38 @@ hipError_t launch_zero_state(const e2d_params& p, const DevBuffers& b, int buf, 
 
 // ---------------------------------------------------------------------------
 // deterministic FP64 sums over the interior: block k reduces rows k, k+B, ...
-// in a fixed order, then one block adds the partials in block order.
+// in a fixed order, then one block adds the partials in block order.  Bound by
+// the memory's latency: a thread adds its values one by one, so it loads
+// kSumAhead of them (times 4 variables) before it adds the first (960
+// wavefronts with 4 loads in flight each read 134 MB in 34 us and 537 MB in
+// 186; with 32 in flight, 22 and 119), and the partials pass through LDS (added
+// from memory one by one they took 30 us, now 4).  The order of the additions
+// is the same.
+constexpr int kSumAhead = 8;
 
 template <class S>
 __global__ __launch_bounds__(256) void k_sums_partial(const Grid g, const S* __restrict__ u, double* partial) {
   __shared__ double red[4][256];
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   for (int j = 2 + blockIdx.x; j <= g.ny + 1; j += gridDim.x)
-    for (int i = 2 + threadIdx.x; i <= g.nx + 1; i += blockDim.x)
+    for (int i0 = 2; i0 <= g.nx + 1; i0 += kSumAhead * 256) {
+      S x[kSumAhead][4];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) acc[v] += static_cast<double>(u[at(g, i, j, v)]);
+      for (int k = 0; k < kSumAhead; ++k) {
+        const int i = i0 + k * 256 + static_cast<int>(threadIdx.x);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[k][v] = S(0);
+        if (i0 + k * 256 <= g.nx + 1 && i <= g.nx + 1) {  // the first test is uniform
+#pragma unroll
+          for (int v = 0; v < 4; ++v) x[k][v] = u[at(g, i, j, v)];
+        }
+      }
+      // a zero in the place of a column past the last leaves a sum as it is (no sum is -0)
+#pragma unroll
+      for (int k = 0; k < kSumAhead; ++k)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[v] += static_cast<double>(x[k][v]);
+    }
 #pragma unroll
   for (int v = 0; v < 4; ++v) red[v][threadIdx.x] = acc[v];
   __syncthreads();
@@ -1243,15 +1279,19 @@ __global__ __launch_bounds__(256) void k_sums_partial(const Grid g, const S* __r
   if (threadIdx.x < 4) partial[blockIdx.x * 4 + threadIdx.x] = red[threadIdx.x][0];
 }
 
-__global__ void k_sums_final(const double* partial, int nb, double* out) {
+__global__ __launch_bounds__(256) void k_sums_final(const double* partial, double* out) {
+  __shared__ double p[kSumBlocks * 4];
+  for (int t = threadIdx.x; t < kSumBlocks * 4; t += 256) p[t] = partial[t];
+  __syncthreads();
   if (threadIdx.x < 4) {
     double s = 0.0;
-    for (int k = 0; k < nb; ++k) s += partial[k * 4 + threadIdx.x];
+#pragma unroll 16
+    for (int k = 0; k < kSumBlocks; ++k) s += p[k * 4 + threadIdx.x];
     out[threadIdx.x] = s;
   }
 }
 
-hipError_t launch_sums(const e2d_params& p, const DevBuffers& b, int buf, double* d_out4, hipStream_t s) {
+hipError_t launch_sums(const e2d_params& p, const DevBuffers& b, int buf, double* out4, hipStream_t s) {
   const Grid g = make_grid(p, b);
   if (state_elem_bytes(p.precision) == 8)
     hipLaunchKernelGGL(k_sums_partial<double>, dim3(kSumBlocks), dim3(256), 0, s, g,
@@ -1259,7 +1299,7 @@ hipError_t launch_sums(const e2d_params& p, const DevBuffers& b, int buf, double
   else
     hipLaunchKernelGGL(k_sums_partial<float>, dim3(kSumBlocks), dim3(256), 0, s, g,
                        static_cast<const float*>(b.u[buf]), b.partial);
-  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(64), 0, s, b.partial, kSumBlocks, d_out4);
+  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(256), 0, s, b.partial, out4);
   return hipGetLastError();
 }
 
