@@ -645,22 +645,31 @@ int ensure_adjoint_scratch(e2d_ctx* c) {
   return E2D_OK;
 }
 
-int adjoint_step(e2d_ctx* c, int buf, double dt, const double* lam_in, double* lam_out) {
+// adjoint step at the state in `state` (its ghost cells are filled)
+int adjoint_step(e2d_ctx* c, void* state, double dt, const double* lam_in, double* lam_out) {
+  e2d::DevBuffers b = c->b;
+  b.u[0] = state;
   HIP_TRY(timed(c, E2D_TIMER_GODUNOV,
-                [&] { return e2d::launch_adjoint_step(c->p, c->b, buf, dt, lam_in, lam_out, c->adj, c->stream); }));
+                [&] { return e2d::launch_adjoint_step(c->p, b, 0, dt, lam_in, lam_out, c->adj, c->stream); }));
   return E2D_OK;
 }
 
-// steps n -> n+1 with a given dt (the forward of godunov_unsplit)
-int forward_step(e2d_ctx* c, int n, double dt) {
-  e2d::StepCfg cfg;
-  cfg.buf_in = n % 2;
-  cfg.buf_out = 1 - cfg.buf_in;
-  cfg.dt_host = dt;
-  HIP_TRY(e2d::launch_fused_step(c->p, c->b, cfg, c->stream));
-  return E2D_OK;
+// the device memory of a state: in place of the context's buffers 0 and 1, the
+// states at `in` and `out`
+e2d::DevBuffers with_states(const e2d_ctx* c, void* in, void* out) {
+  e2d::DevBuffers b = c->b;
+  b.u[0] = in;
+  b.u[1] = out;
+  return b;
 }
 
+// Steps of a rollout run between states wherever they lie: the context's two
+// buffers, which the steps ping-pong between, and the snapshots.  A step that
+// ends at a state to keep writes it into its snapshot, and steps from a kept
+// state read it there, so no state is copied.  A state's memory holds what a
+// step reads of it: the interior (ghost cells are rebuilt from it) and the
+// corner ghost cells, which no step writes and which differ between the two
+// buffers; a snapshot gets those of its state's buffer.
 struct Rollout {
   e2d_ctx* c;
   int n0;
@@ -672,35 +681,35 @@ struct Rollout {
   int cur = 0;
   std::vector<int> free_slots;
   int64_t nfwd = 0;
-  // step whose state each buffer holds (-1: none of this rollout).  A step
-  // leaves its input in place (only ghost cells, which every consumer
-  // rebuilds from the interior, are rewritten), so after advancing to k the
-  // other buffer still holds k-1 and a restore of a held state is skipped.
-  int held[2] = {-1, -1};
+  bool start_in_buffer = false;  // buffer n0 % 2 still holds the starting state
 
   // snapshots already stored by e2d_rollout_forward: (step, slot) of the
   // first descent, consumed in order
   std::vector<std::pair<int, int>> pre;
 
-  int buf_of(int k) const { return (n0 + k) % 2; }
-  int save(int slot, int k) {
-    HIP_TRY(hipMemcpyAsync(c->snapshots[slot], c->b.u[buf_of(k)], state_bytes(c), hipMemcpyDeviceToDevice,
-                           c->stream));
+  void* buffer_of(int k) const { return c->b.u[(n0 + k) % 2]; }
+  // step k -> k+1 from the state at `from` to `to` (the forward of godunov_unsplit)
+  int step(int k, void* from, void* to) {
+    e2d::StepCfg cfg;
+    cfg.dt_host = dts[k];
+    HIP_TRY(e2d::launch_fused_step(c->p, with_states(c, from, to), cfg, c->stream));
+    if (to == buffer_of(0)) start_in_buffer = false;
+    ++nfwd;
     return E2D_OK;
   }
-  int restore(int slot, int k) {
-    if (held[buf_of(k)] == k) return E2D_OK;
-    HIP_TRY(hipMemcpyAsync(c->b.u[buf_of(k)], c->snapshots[slot], state_bytes(c), hipMemcpyDeviceToDevice,
-                           c->stream));
-    held[buf_of(k)] = k;
+  // step k -> k+1 from `from` into snapshot `slot`
+  int step_to_snapshot(int k, void* from, int slot) {
+    if (int rc = step(k, from, c->snapshots[slot])) return rc;
+    HIP_TRY(e2d::launch_copy_corners(c->p, with_states(c, buffer_of(k + 1), c->snapshots[slot]), c->stream));
     return E2D_OK;
   }
-  int advance(int from, int to) {
-    for (int k = from; k < to; ++k) {
-      if (int rc = forward_step(c, n0 + k, dts[k])) return rc;
-      held[buf_of(k + 1)] = k + 1;
-      ++nfwd;
+  // state a, at `from`, advanced to step k in the buffers; where it then lies
+  int advance(int a, int k, void* from, void** at) {
+    for (int i = a; i < k; ++i) {
+      if (int rc = step(i, from, buffer_of(i + 1))) return rc;
+      from = buffer_of(i + 1);
     }
+    *at = from;
     return E2D_OK;
   }
   // lam <- J_a^T ... J_{b-1}^T lam, with the state of step a in snapshot `slot`
@@ -709,9 +718,9 @@ struct Rollout {
     const int s = static_cast<int>(free_slots.size());
     if (l == 1 || s == 0) {
       for (int k = b - 1; k >= a; --k) {
-        if (int rc = restore(slot, a)) return rc;
-        if (int rc = advance(a, k)) return rc;
-        if (int rc = adjoint_step(c, buf_of(k), dts[k], lam[cur], lam[1 - cur])) return rc;
+        void* at = nullptr;
+        if (int rc = advance(a, k, c->snapshots[slot], &at)) return rc;
+        if (int rc = adjoint_step(c, at, dts[k], lam[cur], lam[1 - cur])) return rc;
         cur = 1 - cur;
       }
       return E2D_OK;
@@ -722,9 +731,9 @@ struct Rollout {
     if (!pre.empty() && pre.front() == std::make_pair(a + m, mine)) {
       pre.erase(pre.begin());  // recorded by the forward
     } else {
-      if (int rc = restore(slot, a)) return rc;
-      if (int rc = advance(a, a + m)) return rc;
-      if (int rc = save(mine, a + m)) return rc;
+      void* at = nullptr;
+      if (int rc = advance(a, a + m - 1, c->snapshots[slot], &at)) return rc;
+      if (int rc = step_to_snapshot(a + m - 1, at, mine)) return rc;
     }
     if (int rc = reverse(a + m, b, mine)) return rc;
     free_slots.push_back(mine);
@@ -756,7 +765,7 @@ int e2d_adjoint_step(e2d_ctx* c, int buf, double dt, const double* lam_in, doubl
   if (!lam_in || !lam_out) return fail(E2D_ERR_ARG, "field pointer is NULL");
   if (!(dt > 0.0)) return fail(E2D_ERR_ARG, "dt must be > 0");
   if (int rc = ensure_adjoint_scratch(c)) return rc;
-  return adjoint_step(c, buf, dt, lam_in, lam_out);
+  return adjoint_step(c, c->b.u[buf], dt, lam_in, lam_out);
 }
 
 int e2d_adjoint_rollout(e2d_ctx* c, int nStep0, int nsteps, const double* dts, int nsnap, const double* lam_n,
@@ -796,16 +805,16 @@ int e2d_adjoint_rollout(e2d_ctx* c, int nStep0, int nsteps, const double* dts, i
   Rollout r{c, nStep0, dts, {lam_0, c->lam_tmp}};
   for (int k = nsnap - 1; k >= 1; --k) r.free_slots.push_back(k);
   if (recorded) {
-    // snapshot 0 and the first descent's snapshots hold their states; the
-    // buffers are not trusted (the caller may have stepped since)
+    // snapshot 0 and the first descent's snapshots hold their states
     r.pre = first_descent(nsteps, nsnap);
   } else {
-    r.held[r.buf_of(0)] = 0;
-    if (int rc = r.save(0, 0)) return rc;
+    HIP_TRY(hipMemcpyAsync(c->snapshots[0], r.buffer_of(0), state_bytes(c), hipMemcpyDeviceToDevice, c->stream));
   }
+  r.start_in_buffer = true;  // a recording has been compared with it
   if (int rc = r.reverse(0, nsteps, 0)) return rc;
   if (r.cur == 1) HIP_TRY(hipMemcpyAsync(lam_0, c->lam_tmp, field_bytes(c), hipMemcpyDeviceToDevice, c->stream));
-  if (int rc = r.restore(0, 0)) return rc;
+  if (!r.start_in_buffer)
+    HIP_TRY(hipMemcpyAsync(r.buffer_of(0), c->snapshots[0], state_bytes(c), hipMemcpyDeviceToDevice, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   if (n_forward) *n_forward = r.nfwd;
   return E2D_OK;
@@ -828,14 +837,25 @@ int e2d_rollout_forward(e2d_ctx* c, int nStep0, int nsteps, const double* dts, i
   }
   const std::vector<std::pair<int, int>> plan = first_descent(nsteps, nsnap);
   Rollout r{c, nStep0, dts, {nullptr, nullptr}};
-  if (int rc = r.save(0, 0)) return rc;
+  HIP_TRY(hipMemcpyAsync(c->snapshots[0], r.buffer_of(0), state_bytes(c), hipMemcpyDeviceToDevice, c->stream));
   size_t next = 0;
+  void* at = r.buffer_of(0);
   for (int k = 0; k < nsteps; ++k) {
-    if (int rc = forward_step(c, nStep0 + k, dts[k])) return rc;
-    if (next < plan.size() && plan[next].first == k + 1) {
-      if (int rc = r.save(plan[next].second, k + 1)) return rc;
-      ++next;
+    const bool keep = next < plan.size() && plan[next].first == k + 1;
+    if (keep && k + 1 <= nsteps - 3) {
+      if (int rc = r.step_to_snapshot(k, at, plan[next].second)) return rc;
+      at = c->snapshots[plan[next].second];
+    } else {
+      // the last three states pass through the buffers, so that these end up as
+      // separate steps leave them (the last state's ghost cells are those that
+      // the state two steps before it was given in the same buffer)
+      if (int rc = r.step(k, at, r.buffer_of(k + 1))) return rc;
+      at = r.buffer_of(k + 1);
+      if (keep)
+        HIP_TRY(hipMemcpyAsync(c->snapshots[plan[next].second], at, state_bytes(c), hipMemcpyDeviceToDevice,
+                               c->stream));
     }
+    if (keep) ++next;
   }
   c->rec.valid = true;
   c->rec.n0 = nStep0;

@@ -67,6 +67,8 @@ hipError_t launch_fused_step(const e2d_params& p, const DevBuffers& b, const Ste
 hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c,
                                     hipStream_t s);
 hipError_t launch_boundaries(const e2d_params& p, const DevBuffers& b, int buf, hipStream_t s);
+// the 16 corner ghost cells of buffer 0 of b, which no step writes, to buffer 1
+hipError_t launch_copy_corners(const e2d_params& p, const DevBuffers& b, hipStream_t s);
 // atomic max of the CFL rate over the compute_dt window of buffer buf into invDt slot `slot`
 hipError_t launch_max_invdt(const e2d_params& p, const DevBuffers& b, int buf, int slot, hipStream_t s);
 // the same maximum as one value per block, out[0 .. *nblocks) (at most

@@ -1023,6 +1023,24 @@ hipError_t launch_boundaries(const e2d_params& p, const DevBuffers& b, int buf, 
   return with_precision(p.precision, [&](auto pol) { return boundaries<decltype(pol)>(p, b, buf, s); });
 }
 
+// one wavefront: thread t is variable t / 16 of corner cell t % 16
+template <class S>
+__global__ __launch_bounds__(64) void k_copy_corners(const Grid g, const S* __restrict__ from, S* __restrict__ to) {
+  const int t = threadIdx.x;
+  const int x = t & 3, y = (t >> 2) & 3;
+  const int64_t o = at(g, x < 2 ? x : g.nx + x, y < 2 ? y : g.ny + y, t >> 4);
+  to[o] = from[o];
+}
+
+hipError_t launch_copy_corners(const e2d_params& p, const DevBuffers& b, hipStream_t s) {
+  return with_precision(p.precision, [&](auto pol) {
+    using S = typename decltype(pol)::S;
+    hipLaunchKernelGGL(k_copy_corners<S>, dim3(1), dim3(64), 0, s, make_grid(p, b), static_cast<const S*>(b.u[0]),
+                       static_cast<S*>(b.u[1]));
+    return hipGetLastError();
+  });
+}
+
 // ---------------------------------------------------------------------------
 // compute_dt reduction: max CFL rate over [2, nx] x [2, ny] (0-based)
 
