@@ -125,7 +125,7 @@ E2D_HDI void cons_to_prim_adj(const Hydro<T>& h, const T u[4], const T qb[4], T 
   rho_b += pa_b * gm1 * eint + pb_b * h.smallp;
   const T eint_b = pa_b * gm1 * rho;
   const T e0_b = eint_b, kin_b = -eint_b;
-  const T irho = M::div(T(1), rho);
+  const T irho = M::inv(rho);
   ub[1] += e0_b * irho;
   rho_b -= e0_b * e0 * irho;
   vx_b += kin_b * vx;
@@ -180,7 +180,7 @@ E2D_HDI void trace_sources_adj(const Hydro<T>& h, const T q[4], const T dqx[4],
     dqxb[k] += -u * sb[k];
     dqyb[k] += -v * sb[k];
   }
-  const T ir = M::div(T(1), r);
+  const T ir = M::inv(r);
   dqxb[1] += -sb[2] * ir;
   dqyb[1] += -sb[3] * ir;
   const T dv_b = -sb[0] * r - sb[1] * h.gamma0 * p;
@@ -276,9 +276,9 @@ E2D_HDI T newton_step_adj(const Hydro<T>& h, T pk, T cl, T cr, T pl, T pr,
     pk_b -= delp_b;
   const T m_b = t_b * (usl - usr);
   const T usl_b = t_b * m, usr_b = -t_b * m;
-  const T iS = M::div(T(1), S), iwwl = M::div(T(1), wwl), iwwr = M::div(T(1), wwr);
-  const T idzl = M::div(T(1), dzl), idzr = M::div(T(1), dzr);
-  const T ipl = M::div(T(1), pl), ipr = M::div(T(1), pr);
+  const T iS = M::inv(S), iwwl = M::inv(wwl), iwwr = M::inv(wwr);
+  const T idzl = M::inv(dzl), idzr = M::inv(dzr);
+  const T ipl = M::inv(pl), ipr = M::inv(pr);
   const T pm_b = m_b * iS, s_b = -m_b * m * iS;
   const T zr_b = pm_b * zl + s_b, zl_b = pm_b * zr + s_b;
   // usl = ul - (pk - pl)/wwl ; usr = ur + (pk - pr)/wwr
@@ -330,12 +330,14 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
   const T den = wl0 + wr0;
   const T p0r = M::div(num, den);
   const T p0 = fmax2(p0r, T(0.0));
-  T ps = p0;
+  T ps = p0, p1 = p0, p2 = p0;  // p_1 and p_2 are kept for the reverse
   bool more = true;
   int K = 0;
   for (; K < h.niter && more; ++K) {
     bool tt;
     ps = newton_step<M>(h, ps, cl, cr, pl, pr, ul, ur, more, tt);
+    p1 = K == 0 ? ps : p1;
+    p2 = K <= 1 ? ps : p2;
   }
   const T xlf = M::div(g6 * (ps - pl), pl), xrf = M::div(g6 * (ps - pr), pr);
   const T wl = M::sqrt(cl * (T(1.0) + xlf));
@@ -388,8 +390,8 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
   gs[3] = right ? ql[3] : qr[3];
 
   // ---- reverse (derivative arithmetic with one reciprocal per denominator)
-  const T iro = M::div(T(1), ro), irs = M::div(T(1), rs);
-  const T ipl = M::div(T(1), pl), ipr = M::div(T(1), pr);
+  const T iro = M::inv(ro), irs = M::inv(rs);
+  const T ipl = M::inv(pl), ipr = M::inv(pr);
   T gb[4] = {T(0.0), T(0.0), T(0.0), T(0.0)};
   godunov_flux_adj(h, gs, fb, gb);
   if (right)
@@ -414,7 +416,7 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
     ps_b += gb[1] * frac;
     po_b += gb[1] * (T(1.0) - frac);
     // frac = 0.5 (1 + sum/scr)
-    const T iscr = M::div(T(1), scr);
+    const T iscr = M::inv(scr);
     T sum_b = frac_b * T(0.5) * iscr;
     const T scr_b = -frac_b * T(0.5) * sum * (iscr * iscr);
     T dif_b = T(0.0);
@@ -438,13 +440,13 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
     uo_b += s_uo_b * sg;
     // cs = max(smallc, sqrt|g ps / rs|)
     if (!(h.smallc > cs_r) && cs_r > T(0.0)) {
-      const T X_b = cs_b * T(0.5) * M::div(T(1), cs_r) * sgn(X);
+      const T X_b = cs_b * T(0.5) * M::inv(cs_r) * sgn(X);
       ps_b += X_b * g * irs;
       rs_b -= X_b * g * ps * (irs * irs);
     }
     // co = max(smallc, sqrt|g po / ro|)
     if (!(h.smallc > co_r) && co_r > T(0.0)) {
-      const T Y_b = co_b * T(0.5) * M::div(T(1), co_r) * sgn(Y);
+      const T Y_b = co_b * T(0.5) * M::inv(co_r) * sgn(Y);
       po_b += Y_b * g * iro;
       ro_b -= Y_b * g * po * (iro * iro);
     }
@@ -452,14 +454,14 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
   // rs = max(ro / (1 + ro (po - ps) / wo^2), smallr)
   if (rs_r > h.smallr) {
     const T rsr_b = rs_b;
-    const T iD = M::div(T(1), D);
+    const T iD = M::inv(D);
     ro_b += rsr_b * iD;
     const T E_b = -rsr_b * ro * (iD * iD);
-    const T iw2 = M::div(T(1), wo * wo);
+    const T iw2 = M::inv(wo * wo);
     ro_b += E_b * (po - ps) * iw2;
     po_b += E_b * ro * iw2;
     ps_b -= E_b * ro * iw2;
-    wo_b -= E_b * T(2.0) * E * M::div(T(1), wo);
+    wo_b -= E_b * T(2.0) * E * M::inv(wo);
   }
   T rl_b = T(0.0), ul_b = T(0.0), pl_b = T(0.0), wl_b = T(0.0);
   T rr_b = T(0.0), ur_b = T(0.0), pr_b = T(0.0), wr_b = T(0.0);
@@ -478,7 +480,7 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
   ul_b += T(0.5) * us_b;
   ur_b += T(0.5) * us_b;
   const T a_b = T(0.5) * us_b, b_b = -T(0.5) * us_b;
-  const T iwl = M::div(T(1), wl), iwr = M::div(T(1), wr);
+  const T iwl = M::inv(wl), iwr = M::inv(wr);
   pl_b += a_b * iwl;
   ps_b -= a_b * iwl;
   wl_b -= a_b * a_us * iwl;
@@ -501,18 +503,18 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
     ps_b += x_b * g6 * ipr;
     pr_b += -x_b * g6 * ps * (ipr * ipr);
   }
-  // Newton iterations, last to first (p_k recomputed from p_0)
+  // Newton iterations, last to first (p_k past the kept ones recomputed from p_2)
   T p_b = ps_b;
   for (int k = K - 1; k >= 0; --k) {
-    T pk = p0;
+    T pk = k == 0 ? p0 : (k == 1 ? p1 : p2);
     bool cv, tt;
-    for (int j = 0; j < k; ++j) pk = newton_step<M>(h, pk, cl, cr, pl, pr, ul, ur, cv, tt);
+    for (int j = 2; j < k; ++j) pk = newton_step<M>(h, pk, cl, cr, pl, pr, ul, ur, cv, tt);
     p_b = newton_step_adj<M>(h, pk, cl, cr, pl, pr, ul, ur, p_b, cl_b, cr_b, pl_b, pr_b, ul_b, ur_b);
   }
   // p0 = max(num/den, 0)
   T wl0_b = T(0.0), wr0_b = T(0.0);
   if (p0r > T(0.0)) {
-    const T iden = M::div(T(1), den);
+    const T iden = M::inv(den);
     const T num_b = p_b * iden;
     const T den_b = -p_b * p0r * iden;
     wr0_b += num_b * pl + num_b * wl0 * (ul - ur) + den_b;
@@ -522,8 +524,8 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
     ul_b += num_b * wl0 * wr0;
     ur_b -= num_b * wl0 * wr0;
   }
-  cl_b += wl0_b * T(0.5) * M::div(T(1), wl0);
-  cr_b += wr0_b * T(0.5) * M::div(T(1), wr0);
+  cl_b += wl0_b * T(0.5) * M::inv(wl0);
+  cr_b += wr0_b * T(0.5) * M::inv(wr0);
   // c = g p r
   pl_b += cl_b * g * rl;
   rl_b += cl_b * g * pl;

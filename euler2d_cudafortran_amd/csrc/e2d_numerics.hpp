@@ -55,6 +55,7 @@ struct Hydro {
 // quotient); policies without one leave inv unused.  recip(b) is such a
 // reciprocal of b, and recip_near(b, r0) one from a start r0 within about
 // 2^-50 of 1/b (one Newton step); both return 0 where div_inv ignores them.
+// inv(b) is 1 / b for derivative arithmetic: within half an ulp and 2^-20 of one.
 // quot_gt(a, d, tol, h) is div(a, d) > tol for a >= 0 (or NaN) and d > 0,
 // h being half an ulp of tol; a policy may decide it without the quotient.
 struct ExactMath {
@@ -73,6 +74,8 @@ struct ExactMath {
   static E2D_HDI T div_inv(T a, T b, T) { return div(a, b); }
   template <class T>
   static E2D_HDI T recip(T) { return T(0); }
+  template <class T>
+  static E2D_HDI T inv(T b) { return T(1) / b; }
   template <class T>
   static E2D_HDI T recip_near(T, T) { return T(0); }
   template <class T>
@@ -93,6 +96,7 @@ struct FastMath {
   }
   static __device__ __forceinline__ float div_inv(float a, float, float r) { return a * r; }
   static __device__ __forceinline__ float recip(float b) { return __builtin_amdgcn_rcpf(b); }
+  static __device__ __forceinline__ float inv(float b) { return recip(b); }
   static __device__ __forceinline__ float recip_near(float b, float) { return recip(b); }
   static __device__ __forceinline__ bool quot_gt(float a, float d, float tol, float) { return div(a, d) > tol; }
 };
@@ -125,6 +129,7 @@ struct RangedMath {
     const float r = __builtin_amdgcn_rcpf(b);
     return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
   }
+  static __device__ __forceinline__ float inv(float b) { return recip(b); }
   // the start is not used: v_rcp_f32 and one step are as short
   static __device__ __forceinline__ float recip_near(float b, float) { return recip(b); }
   static __device__ __forceinline__ float div_inv(float a, float b, float r) {
@@ -171,6 +176,7 @@ struct RangedMath {
     const double e = __builtin_fma(-b, r, 1.0);
     return __builtin_fma(r, __builtin_fma(e, e, e), r);
   }
+  static __device__ __forceinline__ double inv(double b) { return recip(b); }
   // one Newton step from r0 = 1/b (1 + e0): error e0^2 and the step's
   // rounding, as close as recip(b) once |e0| is below about 2^-50
   static __device__ __forceinline__ double recip_near(double b, double r0) {
