@@ -25,6 +25,7 @@
 // each step's contribution is added to lam in double.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -856,6 +857,293 @@ __global__ __launch_bounds__(64 * kAdjWaves) __attribute__((amdgpu_waves_per_eu(
   adj_march_gather_body<P>(a);
 }
 
+// k_adj_march_gather's passes on tiles.  A workgroup takes a strip of 64 columns
+// (58 gathered) and R completed rows [ra, ra + R), one row a wavefront: R + 2
+// wavefronts, wavefront w on row r = ra - 1 + w, whose rows meet in LDS.  Each
+// forms its row's primitives (the outer two also those of the rows beyond), then
+// slopes, sources and face states and the x-faces' Riemann adjoint, then the
+// Riemann adjoint of the y-face below its row (the row below's upper state from
+// LDS, that state's bar back to it), then completes its row and forms its
+// limiter adjoints, and with the parts of the rows below and above (LDS) the
+// cell's bar of u.  The first and the last row of the tile miss a part that
+// another tile forms and go to the seam buffer, as there.  The input's ghost
+// cells are formed on load and written back (no fill before this kernel).
+// The values and their order are k_adj_march_gather's, so the bits are the same.
+// us per adjoint step against the march, all kernels: 64^2 FP64 72.1, 30.0;
+// 256^2 84.1, 36.1; 512^2 81.8, 72.6; 512^2 FP32 65.2, 50.1 (a grid that small
+// gives the march one wavefront per SIMD or fewer, each with a chain of 6 or
+// more row iterations).
+constexpr int kAdjTileMaxRows = 10;
+// resident wavefronts per SIMD: FP64 takes 155 VGPRs, the float variants 86-88
+template <class T>
+constexpr int adj_tile_waves() {
+  return sizeof(T) == 8 ? 3 : 5;
+}
+// rows of LDS (4 variables x 64 lanes of T): primitives; lower states of the
+// y-faces, then their bars, then plus parts; minus parts; bars of the x-face
+// states (what a wavefront keeps across a Riemann adjoint lies in LDS or is
+// formed again, as that alone takes 153 VGPRs in FP64)
+constexpr int adj_tile_lds_rows(int rows) { return (rows + 4) + (rows + 1) + 3 * rows; }
+
+// cell (i, j) of the state with its ghost cells filled (corners as stored)
+template <class P>
+__device__ __forceinline__ Src filled_cell(const AdjArgs<P>& a, int i, int j, typename P::S raw[4]) {
+  const Src s = ghost_source(a.g, i, j);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    raw[v] = a.u[at(a.g, s.i, s.j, v)];
+    if (v == s.flip) raw[v] = -raw[v];
+  }
+  return s;
+}
+
+template <class P>
+__global__ __launch_bounds__(64 * (kAdjTileMaxRows + 2))
+__attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj_tile(const AdjArgs<P> a) {
+  using S = typename P::S;
+  using T = typename P::T;
+  using U = typename P::U;
+  using M = typename P::M;
+  extern __shared__ __align__(16) unsigned char adj_tile_mem[];
+  const Grid& g = a.g;
+  const int R = a.seg_rows;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = static_cast<int>(threadIdx.x & 63);
+  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
+  const int strip = lb / a.nsegs;
+  int ra, rb;
+  adj_segment_rows(a, lb - strip * a.nsegs, ra, rb);
+  const int nr = rb - ra;
+  const int r = ra - 1 + wave;  // the wavefront's row
+  const int ci = strip * kFusedStripOut + lane - 3;  // column of this lane
+  const int cl = ci < 0 ? 0 : (ci > g.isize - 1 ? g.isize - 1 : ci);
+  const bool cell_col = ci >= 1 && ci <= g.isize - 2;          // the column has completions
+  const bool done_col = lane >= 2 && lane < 62 && cell_col;    // completed on this lane
+  const bool xface = lane >= 2 && lane <= 62 && ci >= 2 && ci <= g.nx + 2;  // face ci-1/2
+  const bool yface = lane >= 2 && lane < 62 && ci >= 2 && ci <= g.nx + 1;
+  const bool gat_col = lane >= 3 && lane <= 60 && ci >= 0 && ci < g.isize;  // gathered on this lane
+  const bool limited = slopes_limited(a.h);
+  const T st = static_cast<T>(a.h.slope_type);
+  const T skip = -T(0);
+  const int left = lane > 0 ? lane - 1 : 0, right = lane < 63 ? lane + 1 : 63;
+  const bool has_row = wave < nr + 2, own_row = wave >= 1 && wave <= nr;
+
+  T* const q_lds = reinterpret_cast<T*>(adj_tile_mem);  // row k: primitives of grid row ra - 2 + k
+  T* const y_lds = q_lds + (R + 4) * 256;               // y-face k, between grid rows ra-1+k and ra+k
+  T* const m_lds = y_lds + (R + 1) * 256;               // minus part of grid row ra + k, for the row below it
+  T* const x_lds = m_lds + R * 256;                     // bars of the x-face states of grid row ra + k
+  T* const qr = q_lds + (wave + 1) * 256 + lane;        // this lane's cell
+  T* const xb = x_lds + (wave - 1) * 512 + lane;
+
+  U dtdxU, dtdyU;
+  step_ratios(a, dtdxU, dtdyU);
+  const T dtdx = static_cast<T>(dtdxU), dtdy = static_cast<T>(dtdyU);
+  auto row = [&](int k) { return k < 0 ? 0 : (k > g.jsize - 1 ? g.jsize - 1 : k); };
+
+  // primitives
+  double lam_r[4] = {0.0, 0.0, 0.0, 0.0};  // zero outside the interior
+  if (has_row) {
+    auto load = [&](int j, T* to) {
+      S raw[4];
+      const Src s = filled_cell(a, cl, row(j), raw);
+      if (s.ghost && cl == ci && row(j) == j) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) const_cast<S*>(a.u)[at(g, ci, j, v)] = raw[v];
+      }
+      T u[4], q[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) u[v] = static_cast<T>(raw[v]);
+      cons_to_prim<T, M>(a.h, u, q);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) to[v * 64] = q[v];
+    };
+    load(r, qr);
+    if (wave == 0) load(r - 1, qr - 256);
+    if (wave == nr + 1) load(r + 1, qr + 256);
+    if (interior(g, ci, r)) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) lam_r[v] = a.lam[at(g, ci, r, v)];
+    }
+  }
+  __syncthreads();
+
+  // the row's slopes and trace sources, from LDS each time they are needed
+  auto trace = [&](T q[4], T dqx[4], T dqy[4], T s[4]) {
+    T xm[4], xp[4], ym[4], yp[4];
+    const T* const rw = qr - lane;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      q[v] = qr[v * 64];
+      xm[v] = rw[v * 64 + left];
+      xp[v] = rw[v * 64 + right];
+      ym[v] = qr[v * 64 - 256];
+      yp[v] = qr[v * 64 + 256];
+    }
+    cell_slopes(a.h, q, xp, xm, yp, ym, dqx, dqy);
+    trace_sources<T, M>(a.h, q, dqx, dqy, s);
+  };
+
+  if (has_row) {
+    T q[4], dqx[4], dqy[4], s[4], f[4];
+    trace(q, dqx, dqy, s);
+    if (wave <= nr) {
+      face_state(a.h, q, dqy, s, dtdy, true, f);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) y_lds[(wave * 4 + v) * 64 + lane] = f[v];
+    }
+    if (own_row) {
+      T xl[4], xr[4], fb[4], xlb[4] = {T(0), T(0), T(0), T(0)}, bxm[4] = {T(0), T(0), T(0), T(0)};
+      bool any = false;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        // 0 + lam and x - 0 give the bits of leaving out the zero terms
+        const double x = (0.0 + lam_r[v]) - from_left<true>(lam_r[v]);
+        fb[v] = static_cast<T>(x * static_cast<double>(dtdxU));
+        any |= (x != 0.0);
+      }
+      face_state(a.h, q, dqx, s, dtdx, true, f);
+      face_state(a.h, q, dqx, s, dtdx, false, xr);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) xl[v] = from_left<true>(f[v]);
+      if (xface && r >= 2 && r <= g.ny + 1 && any) riemann_two_shock_adj<M>(a.h, xl, xr, fb, xlb, bxm);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        xb[v * 64] = bxm[v];
+        xb[v * 64 + 256] = from_right<true>(xlb[v]);
+      }
+    }
+  }
+  __syncthreads();
+
+  T bym[4] = {T(0), T(0), T(0), T(0)};
+  if (has_row && wave >= 1) {
+    T* const yf = y_lds + (wave - 1) * 256 + lane;
+    T fl[4], fr[4], fb[4], ylb[4] = {T(0), T(0), T(0), T(0)};
+    bool any = false;
+    {
+      double lam_p[4] = {0.0, 0.0, 0.0, 0.0};
+      if (interior(g, ci, r - 1)) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) lam_p[v] = a.lam[at(g, ci, r - 1, v)];
+      }
+      if (interior(g, ci, r)) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) lam_r[v] = a.lam[at(g, ci, r, v)];
+      }
+      T q[4], dqx[4], dqy[4], s[4];
+      trace(q, dqx, dqy, s);
+      face_state(a.h, q, dqy, s, dtdy, false, fr);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const double y = (0.0 + lam_r[v]) - lam_p[v];
+        fb[v] = static_cast<T>(y * static_cast<double>(dtdyU));
+        any |= (y != 0.0);
+        fl[v] = yf[v * 64];
+      }
+    }
+    if (yface && r >= 2 && r <= g.ny + 2 && any) riemann_y_adj<M>(a.h, fl, fr, fb, ylb, bym);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) yf[v * 64] = ylb[v];
+  }
+  __syncthreads();
+
+  // completion and limiter adjoints of the row (k_adj_march_gather's row k)
+  T qbx[4], y0f[4], ypk[4], ymf[4];
+  if (own_row) {
+    T* const yf = y_lds + wave * 256 + lane;  // the y-face above: the bar of the row's upper state
+    T q[4], qbar[4] = {T(0), T(0), T(0), T(0)}, dxb[4] = {T(0), T(0), T(0), T(0)}, dyb[4] = {T(0), T(0), T(0), T(0)};
+    {
+      T dqx[4], dqy[4], s[4], ylb[4], bxm[4], bxp[4];
+      trace(q, dqx, dqy, s);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        ylb[v] = yf[v * 64];
+        bxm[v] = xb[v * 64];
+        bxp[v] = xb[v * 64 + 256];
+      }
+      if (done_col) {
+        bool any = false;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) any |= (bxm[v] != T(0)) | (bxp[v] != T(0)) | (bym[v] != T(0)) | (ylb[v] != T(0));
+        if (any) {
+          T sb[4] = {T(0), T(0), T(0), T(0)};
+          face_state_adj(a.h, q, dqx, s, dtdx, false, bxm, qbar, dxb, sb);
+          face_state_adj(a.h, q, dqx, s, dtdx, true, bxp, qbar, dxb, sb);
+          face_state_adj(a.h, q, dqy, s, dtdy, false, bym, qbar, dyb, sb);
+          face_state_adj(a.h, q, dqy, s, dtdy, true, ylb, qbar, dyb, sb);
+          trace_sources_adj<M>(a.h, q, dqx, dqy, sb, qbar, dxb, dyb);
+        }
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const bool xv = limited && done_col && dxb[v] != T(0);
+      T xm = T(0), x0 = T(0), xp = T(0);
+      if (xv) limited_slope_adj(st, qr[v * 64 - lane + left], q[v], qr[v * 64 - lane + right], dxb[v], xm, x0, xp);
+      const T lp = from_left<true>(xp), rm = from_right<true>(xm);
+      const bool lv = from_left<true>(static_cast<int>(xv)) != 0;
+      const bool rv = from_right<true>(static_cast<int>(xv)) != 0;
+      qbx[v] = qbar[v];
+      if (limited) {
+        if (lv) qbx[v] += lp;  // left neighbour: this cell is its plus side
+        if (xv) qbx[v] += x0;
+        if (rv) qbx[v] += rm;  // right neighbour: this cell is its minus side
+      }
+      const bool yv = limited && done_col && dyb[v] != T(0);
+      T ym = T(0), y0 = T(0), yp = T(0);
+      if (yv) limited_slope_adj(st, qr[v * 64 - 256], q[v], qr[v * 64 + 256], dyb[v], ym, y0, yp);
+      ymf[v] = yv ? ym : skip;
+      y0f[v] = yv ? y0 : skip;
+      ypk[v] = yv ? yp : skip;
+      yf[v * 64] = ypk[v];
+      m_lds[((wave - 1) * 4 + v) * 64 + lane] = ymf[v];
+    }
+  }
+  __syncthreads();
+
+  if (!own_row || !gat_col) return;
+  if (wave == 1) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      a.seam[seam_at(g, r, 0, v, ci)] = qbx[v];
+      a.seam[seam_at(g, r, 1, v, ci)] = y0f[v];
+      a.seam[seam_at(g, r, 2, v, ci)] = ymf[v];
+    }
+  }
+  if (wave == 2) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) a.seam[seam_at(g, r, 0, v, ci)] = ymf[v];
+  }
+  T acc[4];
+  if (wave > 1) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = (qbx[v] + y_lds[((wave - 1) * 4 + v) * 64 + lane]) + y0f[v];
+  }
+  if (wave == nr) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (wave > 1) a.seam[seam_at(g, r, 1, v, ci)] = acc[v];
+      a.seam[seam_at(g, r, 3, v, ci)] = ypk[v];
+    }
+  } else if (wave > 1) {
+    S raw[4];
+    filled_cell(a, ci, r, raw);
+    T u[4], ub[4] = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      u[v] = static_cast<T>(raw[v]);
+      acc[v] += m_lds[(wave * 4 + v) * 64 + lane];
+    }
+    cons_to_prim_adj<M>(a.h, u, acc, ub);
+    if (interior(g, ci, r)) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) a.out[at(g, ci, r, v)] = a.lam[at(g, ci, r, v)] + static_cast<double>(ub[v]);
+    } else {
+      store4(a.ub, g, ci, r, ub);
+    }
+  }
+}
+
 // The rows k_adj_march_gather leaves unfinished: row 0, row jsize-1, and the
 // first and last row of every segment, from the seam buffer.  Thread row t:
 // 0 -> row 0, 1 -> row jsize-1, 2 + 2s -> first row of segment s, 3 + 2s ->
@@ -1094,6 +1382,31 @@ int gather_seg_rows() {
   return 8;
 }
 
+// Rows per tile of k_adj_tile, or 0 for the march.  Tiles up to 1,500 cells per
+// compute unit in FP64 (about 620^2) and 4,100 in the float variants (1024^2),
+// where the two cross (march against tiles, us per adjoint step with the seam
+// and frame kernels: 512^2 FP64 81.8, 72.6, 768^2 123.9, 131.2; 1024^2 FP32
+// 123.8, 119.8, mixed 110.3, 107.7; 2048^2 FP32 313, 422).  2 rows, whose 4
+// wavefronts spread over the SIMDs, while one round of such tiles holds the
+// grid (128^2 FP64 25.3 us, with 7 rows 40.6); beyond, 7 rows in FP64 and 6 in
+// the float variants, which form less twice (512^2: 72.6 against 80.3 with 2
+// rows; FP32 50.1 against 51.2).  E2D_ADJOINT_TILE_ROWS gives the rows (0: march);
+// E2D_ADJOINT_PASSES=fused or a segment plan of the march selects the march.
+int plan_adjoint_tile(const Grid& g, size_t elem) {
+  const int forced = adj_env("E2D_ADJOINT_TILE_ROWS", -1);
+  if (forced >= 0) return std::min(forced, kAdjTileMaxRows);
+  const int64_t cus = device_cus();
+  if (static_cast<int64_t>(g.nx) * g.ny > (elem == 8 ? 1500 : 4100) * cus) return 0;
+  for (const char* name : {"E2D_ADJOINT_PASSES", "E2D_ADJOINT_SEG_ROWS", "E2D_ADJOINT_SHORT_ROWS",
+                           "E2D_ADJOINT_LONG_PCT", "E2D_ADJOINT_CHUNK"})
+    if (getenv(name)) return 0;
+  const int64_t strips = (g.isize + kFusedStripOut - 1) / kFusedStripOut;
+  const int64_t tiles = strips * ((g.jsize - 2 + 1) / 2);
+  const int64_t round = cus * (elem == 8 ? 4 * adj_tile_waves<double>() : 4 * adj_tile_waves<float>()) / 4;
+  if (tiles <= round) return 2;
+  return elem == 8 ? 7 : 6;
+}
+
 template <class P>
 hipError_t adjoint_step(const e2d_params& p, const DevBuffers& b, int buf, double dt, const double* lam_in,
                         double* lam_out, const AdjointScratch& s, hipStream_t st) {
@@ -1116,11 +1429,24 @@ hipError_t adjoint_step(const e2d_params& p, const DevBuffers& b, int buf, doubl
   a.ub = static_cast<T*>(s.ub);
   a.seam = static_cast<T*>(s.seam);
   a.dt = dt;
-  hipError_t e = launch_boundaries(p, b, buf, st);
-  if (e != hipSuccess) return e;
   const Grid& g = a.g;
   const Passes passes = adjoint_passes(lam_in == lam_out);
-  if (passes == Passes::kSeparate) {
+  const int tile_rows = passes == Passes::kFused ? plan_adjoint_tile(g, sizeof(T)) : 0;
+  if (tile_rows == 0) {
+    const hipError_t e = launch_boundaries(p, b, buf, st);
+    if (e != hipSuccess) return e;
+  }
+  if (tile_rows > 0) {
+    const int nstrips = (g.isize + kFusedStripOut - 1) / kFusedStripOut;
+    a.seg_rows = tile_rows;
+    a.nsegs = (g.jsize - 2 + tile_rows - 1) / tile_rows;
+    a.short_base = g.jsize - 1;
+    a.nshort = 0;
+    a.short_rows = 1;
+    hipLaunchKernelGGL(k_adj_tile<P>, dim3(nstrips * a.nsegs), dim3(64 * (tile_rows + 2)),
+                       adj_tile_lds_rows(tile_rows) * 256 * sizeof(T), st, a);
+    hipLaunchKernelGGL(k_adj_seam<P>, dim3((g.isize + 63) / 64, (2 + 2 * a.nsegs + 3) / 4), dim3(256), 0, st, a);
+  } else if (passes == Passes::kSeparate) {
     hipLaunchKernelGGL(k_adj_prim<P>, dim3((g.isize + 63) / 64, (g.jsize + 3) / 4), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_adj_faces<P>, dim3((g.nx + 1 + 63) / 64, (g.ny + 1 + 3) / 4), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_adj_cells<P>, dim3((g.isize - 2 + 63) / 64, (g.jsize - 2 + 3) / 4), dim3(256), 0, st,

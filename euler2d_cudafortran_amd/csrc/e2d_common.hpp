@@ -79,6 +79,18 @@ inline Hydro<T> make_hydro(const e2d_params& p) {
   return h;
 }
 
+// compute units of the current device (256 on MI355X), per host thread
+inline int device_cus() {
+  thread_local int cus = 0;
+  if (cus == 0) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      cus = 256;
+  }
+  return cus;
+}
+
 struct Grid {
   int nx, ny, isize, jsize;
   int64_t pitch, plane;

@@ -692,18 +692,6 @@ static int fused_seg_rows(int ny, int waves_per_simd = 3) {
   return d < 1 ? 1 : (d > 32 ? 32 : d);
 }
 
-// compute units of the current device (256 on MI355X), per host thread
-static int device_cus() {
-  thread_local int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
-  }
-  return cus;
-}
-
 // resident wavefronts per SIMD of a kernel launched with kWavesPerBlock waves per block
 static int waves_per_simd(const void* kernel) {
   int blocks_per_cu = 0;

@@ -619,3 +619,31 @@ def test_marching_adjoint_equals_separate_passes(gpu_lib, prec, monkeypatch):
             got = res[mode + " in place"]
             assert np.array_equal(got[interior], res["separate"][interior]), f"{mode} in place bc={bc} {nx}x{ny}"
             assert np.array_equal(got[~interior], lam[~interior]), f"{mode} in place ghosts bc={bc} {nx}x{ny}"
+
+
+# a single strip and two (58 columns each), tiles higher than the grid, rows that do not divide
+@pytest.mark.parametrize("rows", [1, 2, 7, 10])
+@pytest.mark.parametrize("nx, ny, bc, st", [(4, 4, (1, 1, 1, 1), 1), (54, 9, (1, 2, 3, 1), 2), (57, 31, (3, 3, 2, 1), 1),
+                                            (121, 23, (2, 1, 3, 3), 0)])
+def test_adjoint_tiles_equal_the_march(gpu_lib, monkeypatch, nx, ny, bc, st, rows):
+    """The adjoint step on tiles gives the marching kernels' lam and leaves the input state with
+    the same filled ghost cells, bit for bit, in every precision."""
+    mask = _interior(nx, ny)
+    rng = np.random.default_rng(nx + rows)
+    u = _smooth_state(nx, ny, 7)
+    u[nx // 2:, :, :2] *= 0.3  # a jump
+    lam = np.where(mask, rng.normal(size=mask.shape), 0.0)
+    lam[:, ny // 2] = 0.0
+    kw = dict(zip(("boundary_type_xmin", "boundary_type_xmax", "boundary_type_ymin", "boundary_type_ymax"), bc))
+    for prec in (e2d.PREC_FP64, e2d.PREC_FP32, e2d.PREC_FP32_NATIVE, e2d.PREC_MIXED):
+        got = []
+        for tile in (0, rows):
+            monkeypatch.setenv("E2D_ADJOINT_TILE_ROWS", str(tile))
+            with e2d.HydroRun(_params(nx, ny, precision=prec, slope_type=st, **kw)) as run:
+                run.upload(0, u)
+                dt = run.compute_dt(0)
+                a, b = run.field_alloc(), run.field_alloc()
+                run.field_upload(a, lam)
+                run.adjoint_step(0, dt, a, b)
+                got.append((run.field_download(b), run.download(0)))
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), prec
