@@ -326,12 +326,24 @@ E2D_HDI T cfl_rate(const Hydro<T>& h, const T u[4]) {
 
 // Limited slope of one variable along one direction (slope_unsplit_hydro_2d,
 // m_utils.f90:298-312): minmod for slope_type 1, MC for 2.  kUnit: st = 1,
-// where st * x is x itself (exactly, signed zeros and NaN included), so the two
-// products are skipped.
+// where st * x is x itself and the centred difference decides nothing: with dl
+// and dr of one sign, rounding is monotone, so |qp - qm| rounded is at least
+// twice the smaller of |dl| and |dr|, and dc has their sign.  What is left is
+// the smaller of them with their sign, zero where dl dr <= 0: 8 instructions
+// instead of 13 in FP64.
+template <class T>
+E2D_HDI T with_sign_of(T magnitude, T sign) { return __builtin_copysign(magnitude, sign); }
+template <>
+E2D_HDI float with_sign_of<float>(float magnitude, float sign) { return __builtin_copysignf(magnitude, sign); }
 template <bool kUnit, class T>
 E2D_HDI T limited_slope_st(T st, T qm, T q0, T qp) {
-  const T dl = kUnit ? (q0 - qm) : st * (q0 - qm);
-  const T dr = kUnit ? (qp - q0) : st * (qp - q0);
+  if constexpr (kUnit && std::is_floating_point<T>::value) {
+    const T dl = q0 - qm, dr = qp - q0;
+    const T lim = with_sign_of(fmin2(fabs_(dl), fabs_(dr)), dl);
+    return (dl * dr) <= T(0) ? T(0) : lim;
+  }
+  const T dl = st * (q0 - qm);
+  const T dr = st * (qp - q0);
   const T dc = T(0.5) * (qp - qm);
   T lim = fmin2(fabs_(dl), fabs_(dr));
   if ((dl * dr) <= T(0)) lim = T(0);
