@@ -419,3 +419,41 @@ def test_tile_rows_vs_march(gpu_lib, monkeypatch, nx, ny, bc, st, rows):
                 got.append((run.download(0), run.download(1), run.invdt))
         (a0, a1, ai), (b0, b1, bi) = got
         assert _same(b0, a0) and _same(b1, a1) and ai == bi, (prec, _diff_report(b0, a0))
+
+
+@pytest.mark.parametrize("prec", [e2d.PREC_FP64, e2d.PREC_FP32, e2d.PREC_FP32_NATIVE, e2d.PREC_MIXED])
+@pytest.mark.parametrize("nx, ny, tile", [(64, 48, 0), (64, 48, 3), (33, 21, 0)])
+def test_skipped_rates_never_set_dt(gpu_lib, monkeypatch, prec, nx, ny, tile):
+    """The device-resident loop forms a cell's CFL rate only where a bound of it reaches the
+    running maximum; the host-driven loop forms every one.  Equal bits of both buffers and the
+    running invDt on states that stretch the bound: flow up to Mach 1e5 (E / rho cancels against
+    the kinetic energy), densities and pressures at and below their floors, and near-maximal
+    rates all over a uniform flow."""
+    monkeypatch.setenv("E2D_TILE_ROWS", str(tile))
+    rng = np.random.default_rng(nx + tile)
+    shape = (nx + 4, ny + 4)
+    for kind in ("fast", "floors", "uniform"):
+        u = np.empty(shape + (4,))
+        if kind == "uniform":
+            u[...] = [1.0, 2.5, 0.3, -0.2]
+            u *= 1 + 1e-6 * rng.uniform(-1, 1, u.shape)
+        else:
+            rho = rng.uniform(0.1, 2, shape) if kind == "fast" else 10.0 ** rng.uniform(-9, 0, shape)
+            vel = 10.0 ** rng.uniform(-3, 2, shape + (2,)) * rng.choice([-1, 1], shape + (2,))
+            p = 10.0 ** rng.uniform(-12 if kind == "floors" else -6, 0, shape)
+            u[..., 0], u[..., 2:] = rho, rho[..., None] * vel
+            u[..., 1] = p / 0.4 + 0.5 * rho * (vel ** 2).sum(-1)
+        res = []
+        for host in (True, False):
+            with e2d.HydroRun(_params(nx, ny, 0, prec)) as run:
+                run.upload(0, u)
+                if host:
+                    run.run_reference_loop(6)
+                    run.compute_dt(0)
+                else:
+                    run.compute_dt(0)
+                    run.make_boundaries(0)
+                    run.run_steps(6)
+                res.append((run.download(0), run.download(1), run.invdt))
+        assert res[0][2] == res[1][2] or (np.isnan(res[0][2]) and np.isnan(res[1][2])), kind
+        assert _same(res[1][0], res[0][0]) and _same(res[1][1], res[0][1]), kind
