@@ -515,15 +515,17 @@ E2D_HDI void two_shock_finish(const Hydro<T>& h, const T ql[4], const T qr[4], c
     spout = ushock;
   }
   const T scr = fmax2(spout - spin, h.smallc + fabs_(spout + spin));
-  // outside the fan the weight is 0 (the upwind state) or 1 (the star state),
-  // which leaves that state as it is: one select for the reference's three
-  T frac = T(0.5) * (T(1) + M::div(spout + spin, scr));
-  if (spout < T(0)) frac = T(0);
-  if (spin > T(0)) frac = T(1);
-  const T rest = T(1) - frac;
-  const T gr = frac * r_star + rest * ro;
-  const T gu = frac * u_star + rest * uo;
-  const T gp = frac * p_star + rest * po;
+  const T frac = T(0.5) * (T(1) + M::div(spout + spin, scr));
+
+  T gr = frac * r_star + (T(1) - frac) * ro;
+  T gu = frac * u_star + (T(1) - frac) * uo;
+  T gp = frac * p_star + (T(1) - frac) * po;
+  if (spout < T(0)) {
+    gr = ro; gu = uo; gp = po;
+  }
+  if (spin > T(0)) {
+    gr = r_star; gu = u_star; gp = p_star;
+  }
   g[0] = gr;
   g[1] = gp;
   g[2] = gu;
