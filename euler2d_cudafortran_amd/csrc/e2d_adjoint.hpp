@@ -69,6 +69,7 @@ struct DualMath {
   static E2D_HDI Dual div_inv(Dual a, Dual b, Dual) { return div(a, b); }
   static E2D_HDI Dual recip(Dual) { return Dual(0.0, 0.0); }
   static E2D_HDI Dual recip_near(Dual, Dual) { return Dual(0.0, 0.0); }
+  static E2D_HDI Dual inv_given(Dual b, Dual) { return div(Dual(1.0, 0.0), b); }
   static E2D_HDI bool quot_gt(Dual a, Dual d, Dual tol, Dual h) { return Base::quot_gt(a.v, d.v, tol.v, h.v); }
 };
 
@@ -136,32 +137,29 @@ E2D_HDI void cons_to_prim_adj(const Hydro<T>& h, const T u[4], const T qb[4], T 
   if (u[0] > h.smallr) ub[0] += rho_b;
 }
 
-// limited_slope(st, qm, q0, qp): bars of (qm, q0, qp) from the bar of the slope
+// limited_slope(st, qm, q0, qp): bars of (qm, q0, qp) from the bar of the slope.
+// The slope is dc where |dc| is the smallest part (ties and uniform states
+// included), else 0 where dl dr <= 0, else the smaller of dl and dr, whose sign
+// dc shares: whichever it is, the bar of that difference is ob itself, so two
+// selects place it and the middle one's bar is minus the sum of the other two.
 template <class T>
 E2D_HDI void limited_slope_adj(T st, T qm, T q0, T qp, T ob, T& qm_b,
                                T& q0_b, T& qp_b) {
   const T dl = st * (q0 - qm);
   const T dr = st * (qp - q0);
   const T dc = T(0.5) * (qp - qm);
-  const T adl = fabs_(dl), adr = fabs_(dr), adc = fabs_(dc);
-  const T lim0 = fmin2(adl, adr);
-  const T lim = ((dl * dr) <= T(0.0)) ? T(0.0) : lim0;
-  const T m_b = (dc >= T(0.0)) ? ob : -ob;
-  T lim_b = T(0.0), adc_b = T(0.0);
-  if (lim < adc)
-    lim_b = m_b;
-  else
-    adc_b = m_b;
-  const T lim0_b = ((dl * dr) <= T(0.0)) ? T(0.0) : lim_b;
-  T adl_b = T(0.0), adr_b = T(0.0);
-  if (adl < adr)
-    adl_b = lim0_b;
-  else
-    adr_b = lim0_b;
-  const T dl_b = adl_b * sgn(dl), dr_b = adr_b * sgn(dr), dc_b = adc_b * sgn(dc);
-  q0_b += st * dl_b - st * dr_b;
-  qm_b += -st * dl_b - T(0.5) * dc_b;
-  qp_b += st * dr_b + T(0.5) * dc_b;
+  const T adl = fabs_(dl), adr = fabs_(dr);
+  const bool opposed = (dl * dr) <= T(0.0);
+  const T lim = opposed ? T(0.0) : fmin2(adl, adr);
+  const bool centred = !(lim < fabs_(dc));
+  const bool left = adl < adr;
+  T x = opposed ? T(0.0) : st * ob;
+  if (centred) x = T(0.5) * ob;
+  const T m = (centred || left) ? x : T(0.0);
+  const T p = (centred || !left) ? x : T(0.0);
+  qm_b -= m;
+  q0_b += m - p;
+  qp_b += p;
 }
 
 template <class T>
@@ -229,18 +227,20 @@ E2D_HDI void godunov_flux_adj(const Hydro<T>& h, const T g[4], const T fb[4], T 
   gb[2] += mass_b * r;
 }
 
-// One Newton iteration of riemann_two_shock from p_k; returns p_{k+1}.  (The
-// square roots keep their zero case here: without it, the FP64 adjoint
-// kernel is scheduled 1.5% slower.)
+// One Newton iteration of riemann_two_shock from p_k; returns p_{k+1}.  Here and
+// in the reverse a root's reciprocal comes with the root (the radicands are
+// positive: 1 + g6 (p - p0) / p0 >= 1 - g6 > 0), which takes a v_rcp_f64 and its
+// step out of each quotient by it and out of each bar.
 template <class M, class T>
 E2D_HDI T newton_step(const Hydro<T>& h, T pk, T cl, T cr, T pl, T pr,
                            T ul, T ur, bool& more, bool& take_t) {
-  const T wwl = M::sqrt(cl * (T(1.0) + M::div(h.gamma6 * (pk - pl), pl)));
-  const T wwr = M::sqrt(cr * (T(1.0) + M::div(h.gamma6 * (pk - pr), pr)));
+  T iwwl, iwwr;
+  const T wwl = M::sqrt_pos_inv(cl * (T(1.0) + M::div(h.gamma6 * (pk - pl), pl)), iwwl);
+  const T wwr = M::sqrt_pos_inv(cr * (T(1.0) + M::div(h.gamma6 * (pk - pr), pr)), iwwr);
   const T zl = M::div(T(2.0) * wwl * wwl * wwl, wwl * wwl + cl);
   const T zr = M::div(T(2.0) * wwr * wwr * wwr, wwr * wwr + cr);
-  const T usl = ul - M::div(pk - pl, wwl);
-  const T usr = ur + M::div(pk - pr, wwr);
+  const T usl = ul - M::div_inv(pk - pl, wwl, iwwl);
+  const T usr = ur + M::div_inv(pk - pr, wwr, iwwr);
   const T t = M::div(zr * zl, zr + zl) * (usl - usr);
   take_t = t > -pk;
   const T delp = take_t ? t : -pk;
@@ -257,12 +257,13 @@ E2D_HDI T newton_step_adj(const Hydro<T>& h, T pk, T cl, T cr, T pl, T pr,
                                T& pr_b, T& ul_b, T& ur_b) {
   const T g6 = h.gamma6;
   const T xl = M::div(g6 * (pk - pl), pl), xr = M::div(g6 * (pk - pr), pr);
-  const T wwl = M::sqrt(cl * (T(1.0) + xl));
-  const T wwr = M::sqrt(cr * (T(1.0) + xr));
+  T iwwl, iwwr;
+  const T wwl = M::sqrt_pos_inv(cl * (T(1.0) + xl), iwwl);
+  const T wwr = M::sqrt_pos_inv(cr * (T(1.0) + xr), iwwr);
   const T dzl = wwl * wwl + cl, dzr = wwr * wwr + cr;
   const T zl = M::div(T(2.0) * wwl * wwl * wwl, dzl);
   const T zr = M::div(T(2.0) * wwr * wwr * wwr, dzr);
-  const T c1 = M::div(pk - pl, wwl), c2 = M::div(pk - pr, wwr);
+  const T c1 = M::div_inv(pk - pl, wwl, iwwl), c2 = M::div_inv(pk - pr, wwr, iwwr);
   const T usl = ul - c1, usr = ur + c2;
   const T S = zr + zl;
   const T m = M::div(zr * zl, S);
@@ -276,7 +277,9 @@ E2D_HDI T newton_step_adj(const Hydro<T>& h, T pk, T cl, T cr, T pl, T pr,
     pk_b -= delp_b;
   const T m_b = t_b * (usl - usr);
   const T usl_b = t_b * m, usr_b = -t_b * m;
-  const T iS = M::inv(S), iwwl = M::inv(wwl), iwwr = M::inv(wwr);
+  const T iS = M::inv(S);
+  iwwl = M::inv_given(wwl, iwwl);
+  iwwr = M::inv_given(wwr, iwwr);
   const T idzl = M::inv(dzl), idzr = M::inv(dzr);
   const T ipl = M::inv(pl), ipr = M::inv(pr);
   const T pm_b = m_b * iS, s_b = -m_b * m * iS;
@@ -324,8 +327,8 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
   const T pr = fmax2(qr[1], prf);
   const T cl = g * pl * rl;
   const T cr = g * pr * rr;
-  const T wl0 = M::sqrt(cl);
-  const T wr0 = M::sqrt(cr);
+  const T wl0 = M::sqrt_pos(cl);
+  const T wr0 = M::sqrt_pos(cr);
   const T num = (wr0 * pl + wl0 * pr) + wl0 * wr0 * (ul - ur);
   const T den = wl0 + wr0;
   const T p0r = M::div(num, den);
@@ -340,17 +343,23 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
     p2 = K <= 1 ? ps : p2;
   }
   const T xlf = M::div(g6 * (ps - pl), pl), xrf = M::div(g6 * (ps - pr), pr);
-  const T wl = M::sqrt(cl * (T(1.0) + xlf));
-  const T wr = M::sqrt(cr * (T(1.0) + xrf));
-  const T a_us = M::div(pl - ps, wl), b_us = M::div(pr - ps, wr);
+  T iwl, iwr;
+  const T wl = M::sqrt_pos_inv(cl * (T(1.0) + xlf), iwl);
+  const T wr = M::sqrt_pos_inv(cr * (T(1.0) + xrf), iwr);
+  const T a_us = M::div_inv(pl - ps, wl, iwl), b_us = M::div_inv(pr - ps, wr, iwr);
+  iwl = M::inv_given(wl, iwl);
+  iwr = M::inv_given(wr, iwr);
   const T us = T(0.5) * (ul + a_us + ur - b_us);
   const bool right = us >= T(0.0);
   const T ro = right ? rl : rr, uo = right ? ul : ur, po = right ? pl : pr, wo = right ? wl : wr;
   const T sg = right ? T(1.0) : -T(1.0);
   const T Y = M::div(g * po, ro);
-  const T co_r = M::sqrt(fabs_(Y));
+  T ico;
+  const T co_r = M::sqrt_pos_inv(fabs_(Y), ico);
   const T co = fmax2(h.smallc, co_r);
-  const T E = M::div(ro * (po - ps), wo * wo);
+  const T iwo = right ? iwl : iwr;
+  const T iw2 = M::recip_near(wo * wo, iwo * iwo);
+  const T E = M::div_inv(ro * (po - ps), wo * wo, iw2);
   const T D = T(1.0) + E;
   const T rs_r = M::div(ro, D);
   const T rs = fmax2(rs_r, h.smallr);
@@ -446,7 +455,7 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
     }
     // co = max(smallc, sqrt|g po / ro|)
     if (!(h.smallc > co_r) && co_r > T(0.0)) {
-      const T Y_b = co_b * T(0.5) * M::inv(co_r) * sgn(Y);
+      const T Y_b = co_b * T(0.5) * M::inv_given(co_r, ico) * sgn(Y);
       po_b += Y_b * g * iro;
       ro_b -= Y_b * g * po * (iro * iro);
     }
@@ -457,11 +466,11 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
     const T iD = M::inv(D);
     ro_b += rsr_b * iD;
     const T E_b = -rsr_b * ro * (iD * iD);
-    const T iw2 = M::inv(wo * wo);
-    ro_b += E_b * (po - ps) * iw2;
-    po_b += E_b * ro * iw2;
-    ps_b -= E_b * ro * iw2;
-    wo_b -= E_b * T(2.0) * E * M::inv(wo);
+    const T iww = M::inv_given(wo * wo, iw2);
+    ro_b += E_b * (po - ps) * iww;
+    po_b += E_b * ro * iww;
+    ps_b -= E_b * ro * iww;
+    wo_b -= E_b * T(2.0) * E * iwo;
   }
   T rl_b = T(0.0), ul_b = T(0.0), pl_b = T(0.0), wl_b = T(0.0);
   T rr_b = T(0.0), ur_b = T(0.0), pr_b = T(0.0), wr_b = T(0.0);
@@ -480,7 +489,6 @@ E2D_HDI void riemann_two_shock_adj(const Hydro<T>& h, const T ql[4], const T qr[
   ul_b += T(0.5) * us_b;
   ur_b += T(0.5) * us_b;
   const T a_b = T(0.5) * us_b, b_b = -T(0.5) * us_b;
-  const T iwl = M::inv(wl), iwr = M::inv(wr);
   pl_b += a_b * iwl;
   ps_b -= a_b * iwl;
   wl_b -= a_b * a_us * iwl;

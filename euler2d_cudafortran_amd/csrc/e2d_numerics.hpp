@@ -56,6 +56,8 @@ struct Hydro {
 // reciprocal of b, and recip_near(b, r0) one from a start r0 within about
 // 2^-50 of 1/b (one Newton step); both return 0 where div_inv ignores them.
 // inv(b) is 1 / b for derivative arithmetic: within half an ulp and 2^-20 of one.
+// inv_given(b, r) is that from a reciprocal r which sqrt_pos_inv or recip_near
+// left: r itself, or 1 / b where the policy leaves none.
 // quot_gt(a, d, tol, h) is div(a, d) > tol for a >= 0 (or NaN) and d > 0,
 // h being half an ulp of tol; a policy may decide it without the quotient.
 struct ExactMath {
@@ -77,6 +79,8 @@ struct ExactMath {
   template <class T>
   static E2D_HDI T inv(T b) { return T(1) / b; }
   template <class T>
+  static E2D_HDI T inv_given(T b, T) { return inv(b); }
+  template <class T>
   static E2D_HDI T recip_near(T, T) { return T(0); }
   template <class T>
   static E2D_HDI bool quot_gt(T a, T d, T tol, T) { return div(a, d) > tol; }
@@ -97,6 +101,7 @@ struct FastMath {
   static __device__ __forceinline__ float div_inv(float a, float, float r) { return a * r; }
   static __device__ __forceinline__ float recip(float b) { return __builtin_amdgcn_rcpf(b); }
   static __device__ __forceinline__ float inv(float b) { return recip(b); }
+  static __device__ __forceinline__ float inv_given(float, float r) { return r; }
   static __device__ __forceinline__ float recip_near(float b, float) { return recip(b); }
   static __device__ __forceinline__ bool quot_gt(float a, float d, float tol, float) { return div(a, d) > tol; }
 };
@@ -130,6 +135,7 @@ struct RangedMath {
     return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
   }
   static __device__ __forceinline__ float inv(float b) { return recip(b); }
+  static __device__ __forceinline__ float inv_given(float, float r) { return r; }
   // the start is not used: v_rcp_f32 and one step are as short
   static __device__ __forceinline__ float recip_near(float b, float) { return recip(b); }
   static __device__ __forceinline__ float div_inv(float a, float b, float r) {
@@ -177,6 +183,7 @@ struct RangedMath {
     return __builtin_fma(r, __builtin_fma(e, e, e), r);
   }
   static __device__ __forceinline__ double inv(double b) { return recip(b); }
+  static __device__ __forceinline__ double inv_given(double, double r) { return r; }
   // one Newton step from r0 = 1/b (1 + e0): error e0^2 and the step's
   // rounding, as close as recip(b) once |e0| is below about 2^-50
   static __device__ __forceinline__ double recip_near(double b, double r0) {

@@ -53,3 +53,15 @@ def test_float_instantiation_against_double(report):
     n, p99, _ = report["riemann_two_shock_f32"]
     assert n >= 4000
     assert p99 <= 1e-4, f"float vs double Riemann adjoint, 99th percentile {p99:.3e}"
+
+
+@pytest.mark.parametrize("dtype", ["double", "float"])
+def test_limiter_adjoint_branches(tmp_path, dtype):
+    # which difference the bar goes to, at ties and uniform states too: exact
+    exe = tmp_path / "limiter_adjoint_check"
+    subprocess.run([shutil.which("g++"), "-O2", "-std=c++17", "-ffp-contract=off", "-o", str(exe),
+                    str(ROOT / "tests" / "limiter_adjoint_check.cpp")], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    m = re.search(rf"{dtype} n=(\d+) bad=(\d+)", out)
+    assert int(m.group(1)) == 2 * 13 ** 3 * 2
+    assert int(m.group(2)) == 0
