@@ -105,14 +105,12 @@ E2D_HDI Hydro<Dual> dual_hydro(const Hydro<T>& h) {
 template <class T>
 E2D_HDI T sgn(T x) { return x >= T(0.0) ? T(1.0) : -T(1.0); }
 
-// cons_to_prim: u -> q (rho, p, vx, vy)
+// cons_to_prim: u -> q (rho, p, vx, vy), from its floored density, its
+// velocities and the energy u[1] (u[0] > smallr exactly where rho is)
 template <class M, class T>
-E2D_HDI void cons_to_prim_adj(const Hydro<T>& h, const T u[4], const T qb[4], T ub[4]) {
-  const T rho = fmax2(u[0], h.smallr);
-  const T vx = M::div(u[2], rho);
-  const T vy = M::div(u[3], rho);
+E2D_HDI void cons_to_prim_adj(const Hydro<T>& h, T rho, T vx, T vy, T energy, const T qb[4], T ub[4]) {
   const T kin = T(0.5) * (vx * vx + vy * vy);
-  const T e0 = M::div(u[1], rho);
+  const T e0 = M::div(energy, rho);
   const T eint = e0 - kin;
   const T gm1 = h.gamma0 - T(1.0);
   const T pa = gm1 * rho * eint;
@@ -134,7 +132,12 @@ E2D_HDI void cons_to_prim_adj(const Hydro<T>& h, const T u[4], const T qb[4], T 
   ub[2] += vx_b * irho;
   ub[3] += vy_b * irho;
   rho_b -= (vx_b * vx + vy_b * vy) * irho;
-  if (u[0] > h.smallr) ub[0] += rho_b;
+  if (rho > h.smallr) ub[0] += rho_b;
+}
+template <class M, class T>
+E2D_HDI void cons_to_prim_adj(const Hydro<T>& h, const T u[4], const T qb[4], T ub[4]) {
+  const T rho = fmax2(u[0], h.smallr);
+  cons_to_prim_adj<M>(h, rho, M::div(u[2], rho), M::div(u[3], rho), u[1], qb, ub);
 }
 
 // limited_slope(st, qm, q0, qp): bars of (qm, q0, qp) from the bar of the slope.

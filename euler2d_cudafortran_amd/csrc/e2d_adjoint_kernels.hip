@@ -549,12 +549,17 @@ __global__ __launch_bounds__(64 * kAdjWaves) void k_adj_gather_march(const AdjAr
 // and jsize-1).  A part that k_adj_gather skips is carried as -0.0, the
 // identity of IEEE addition, so the sums are bit-identical to the unfused
 // passes.
-// E2D_ADJ_LDS_CARRY=1 (default): the fused kernel's row-carried gather values
-// live in per-thread LDS slots (12 values, 24 KB per FP64 workgroup); in
-// registers the FP64 kernel spills 132 B and is 7% slower (835 vs 778 us).
-#ifndef E2D_ADJ_LDS_CARRY
-#define E2D_ADJ_LDS_CARRY 1
-#endif
+// What a row passes to the next iterations and no Riemann adjoint reads lives in
+// per-thread LDS slots: the gather's 12 values, the bars of the row's 3 face
+// states, lam of two rows and the energies of four (36 values, 72 KB per FP64
+// workgroup, two of which fill a compute unit's LDS as its 2 wavefronts per SIMD
+// do its registers).  The cell is then finished without its u and lam from
+// memory, a wait of the row's end.  FP64 takes 252 VGPRs without a spill, the
+// float variants 139-144.  us per adjoint step at 2048^2 with the gather's 12
+// alone, with the bars, and with lam and energies: FP64 504 (100 B spilled), 475,
+// 453; FP32 292, 293, 280; mixed 268, 261, 256.  (The slopes and sources in LDS as
+// well: 477; the float variants at 4 wavefronts per SIMD, 48-88 B spilled: 308,
+// 318.)
 constexpr int kFusedStripOut = 58;
 // Seam buffer: 4 slots of 4 values per completed row and column, indexed by
 // the row (so that the store addresses vary with the marching loop):
@@ -582,16 +587,15 @@ __device__ __forceinline__ void finish_cell(const AdjArgs<P>& a, int ci, int row
   }
 }
 
-// finish_cell with lam of the cell already in registers (zero for ghost cells,
-// where it is not used)
+// finish_cell with the cell's primitives, energy and lam at hand (lam zero for
+// ghost cells, where it is not used)
 template <class P>
-__device__ __forceinline__ void finish_cell_lam(const AdjArgs<P>& a, int ci, int row, const typename P::T qb[4],
-                                                const double lam[4]) {
+__device__ __forceinline__ void finish_cell_at(const AdjArgs<P>& a, int ci, int row, const typename P::T qb[4],
+                                               const typename P::T q[4], typename P::T energy, const double lam[4]) {
   using T = typename P::T;
   const Grid& g = a.g;
-  T u[4], ub[4] = {T(0), T(0), T(0), T(0)};
-  load4(a.u, g, ci, row, u);
-  cons_to_prim_adj<typename P::M>(a.h, u, qb, ub);
+  T ub[4] = {T(0), T(0), T(0), T(0)};
+  cons_to_prim_adj<typename P::M>(a.h, q[0], q[2], q[3], energy, qb, ub);
   if (interior(g, ci, row)) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) a.out[at(g, ci, row, v)] = lam[v] + static_cast<double>(ub[v]);
@@ -643,35 +647,32 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
   prim_at(a, cl, row(ra - 2), qa);
   prim_at(a, cl, row(ra - 1), qb);
   // row r-1, carried: slopes, trace sources and the bars of its xmin, xmax, ymin face states
-  T pdx[4], pdy[4], ps[4], pbxm[4], pbxp[4], pbym[4];
-  // gather, carried: partial sum of the last completed row, its plus part, and
-  // the primitives of row r-2 (in registers, or with E2D_ADJ_LDS_CARRY in
-  // per-thread LDS slots, out of the registers during the Riemann adjoints)
-#if E2D_ADJ_LDS_CARRY
+  T pdx[4], pdy[4], ps[4];
+  // carried in LDS: partial sum of the last completed row, its plus part, the
+  // primitives of row r-2, and row r-1's face bars
   constexpr int kThreads = 64 * kAdjWaves;
-  __shared__ __align__(16) unsigned char carry_raw[12 * sizeof(T) * kThreads];
-  T* const carry = reinterpret_cast<T*>(carry_raw) + threadIdx.x;
+  __shared__ T carry_raw[24 * kThreads];
+  T* const carry = carry_raw + threadIdx.x;
   auto acc = [&](int v) -> T& { return carry[v * kThreads]; };
   auto ypf = [&](int v) -> T& { return carry[(4 + v) * kThreads]; };
   auto qz = [&](int v) -> T& { return carry[(8 + v) * kThreads]; };
-#else
-  T acc_r[4], ypf_r[4], qz_r[4];
-  auto acc = [&](int v) -> T& { return acc_r[v]; };
-  auto ypf = [&](int v) -> T& { return ypf_r[v]; };
-  auto qz = [&](int v) -> T& { return qz_r[v]; };
-#endif
+  auto xm_b = [&](int v) -> T& { return carry[(12 + v) * kThreads]; };
+  auto xp_b = [&](int v) -> T& { return carry[(16 + v) * kThreads]; };
+  auto ym_b = [&](int v) -> T& { return carry[(20 + v) * kThreads]; };
+  // lam of the last two rows by parity, energies u[1] of the last four
+  __shared__ double lam_raw[8 * kThreads];
+  double* const lam_s = lam_raw + threadIdx.x;
+  auto lam_at = [&](int rw, int v) -> double& { return lam_s[((rw & 1) * 4 + v) * kThreads]; };
+  __shared__ T energy_raw[4 * kThreads];
+  T* const energy_s = energy_raw + threadIdx.x;
+  auto energy = [&](int rw) -> T& { return energy_s[(rw & 3) * kThreads]; };
 #pragma unroll
   for (int v = 0; v < 4; ++v) qz(v) = acc(v) = ypf(v) = T(0);
-  // lam of this lane's cell in rows r and r-1, zero outside the interior: one
-  // load per row; the x-faces take the left column's by a lane shift
-  double lam_r[4], lam_p[4] = {0.0, 0.0, 0.0, 0.0};
+  // lam of this lane's cell in row r, zero outside the interior: one load per
+  // row; the x-faces take the left column's by a lane shift
+  double lam_r[4];
   T un[4];  // state of row r+1, loaded an iteration ahead
   load4(a.u, g, cl, row(ra), un);
-  // lam of row r-2 for finish_cell, carried where it keeps the kernel within
-  // 168 VGPRs (3 waves per SIMD): the mixed instantiation, 167 VGPRs.  FP32
-  // would take 173 (2 waves) and FP64 more scratch spills, both slower.
-  constexpr bool kLamPP = std::is_same<M, FastMath>::value;
-  double lam_pp[4] = {0.0, 0.0, 0.0, 0.0};
 
   for (int r = ra - 1; r <= rb; ++r) {
     {
@@ -679,6 +680,7 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) uc[v] = un[v];
       load4(a.u, g, cl, row(r + 2), un);
+      energy(r + 1) = uc[1];
       cons_to_prim<T, M>(a.h, uc, qc);
     }
     {
@@ -712,7 +714,7 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           // 0 + lam and x - 0 give the bits of leaving out the zero terms
-          const double x = (0.0 + lam_r[v]) - lam_p[v];
+          const double x = (0.0 + lam_r[v]) - lam_at(r - 1, v);
           fb[v] = static_cast<T>(x * static_cast<double>(dtdyU));
           any |= (x != 0.0);
         }
@@ -729,6 +731,13 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
         T qbar[4] = {T(0), T(0), T(0), T(0)}, dxb[4] = {T(0), T(0), T(0), T(0)}, dyb[4] = {T(0), T(0), T(0), T(0)};
         if (done_col) {
           bool any = false;
+          T pbxm[4], pbxp[4], pbym[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            pbxm[v] = xm_b(v);
+            pbxp[v] = xp_b(v);
+            pbym[v] = ym_b(v);
+          }
 #pragma unroll
           for (int v = 0; v < 4; ++v)
             any |= (pbxm[v] != T(0)) | (pbxp[v] != T(0)) | (pbym[v] != T(0)) | (ylb[v] != T(0));
@@ -776,10 +785,11 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
             T qfin[4];
 #pragma unroll
             for (int v = 0; v < 4; ++v) qfin[v] = acc(v) + ymf[v];
-            if constexpr (kLamPP)
-              finish_cell_lam(a, ci, ks - 1, qfin, lam_pp);
-            else
-              finish_cell(a, ci, ks - 1, qfin);
+            double lam_pp[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) lam_pp[v] = lam_at(r - 2, v);
+            const T qk[4] = {qz(0), qz(1), qz(2), qz(3)};
+            finish_cell_at(a, ci, ks - 1, qfin, qk, energy(r - 2), lam_pp);
           }
           if (k == ra) {
 #pragma unroll
@@ -837,24 +847,23 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
       pdx[v] = dqx[v];
       pdy[v] = dqy[v];
       ps[v] = s[v];
-      pbxm[v] = bxm[v];
-      pbxp[v] = bxp[v];
-      pbym[v] = bym[v];
+      xm_b(v) = bxm[v];
+      xp_b(v) = bxp[v];
+      ym_b(v) = bym[v];
       qz(v) = qa[v];
       qa[v] = qb[v];
       qb[v] = qc[v];
-      if constexpr (kLamPP) lam_pp[v] = lam_p[v];
-      lam_p[v] = lam_r[v];
+      lam_at(r, v) = lam_r[v];
     }
+    // the slots stay in LDS: without this the compiler keeps them in registers
+    // from one iteration to the next
+    asm volatile("" ::: "memory");
   }
 }
 
 // The FP64 instantiation is held at 2 resident wavefronts per SIMD (the
-// E2D_ADJ_MARCH_MIN_WAVES cap).  The float-arithmetic ones are held at 3 (168
-// VGPRs): left to itself the compiler gives fp32_native and mixed 173-177
-// VGPRs, 2 wavefronts per SIMD, and their adjoint steps take 312 and 323 us
-// at 2048^2 against 284 and 303 us at 3 (with a 28-36 B spill); FP32 fits
-// in 163 either way.
+// E2D_ADJ_MARCH_MIN_WAVES cap; at 3 it would spill 348 B), the float-arithmetic
+// ones at 3.
 template <class P>
 __global__ __launch_bounds__(64 * kAdjWaves) E2D_ADJ_MARCH_ATTR void k_adj_march_gather(const AdjArgs<P> a) {
   adj_march_gather_body<P>(a);
@@ -1396,8 +1405,8 @@ int gather_seg_rows() {
 // Rows per tile of k_adj_tile, or 0 for the march.  Tiles up to 1,500 cells per
 // compute unit in FP64 (about 620^2) and 4,100 in the float variants (1024^2),
 // where the two cross (march against tiles, us per adjoint step with the seam
-// and frame kernels: 512^2 FP64 81.8, 72.6, 768^2 123.9, 131.2; 1024^2 FP32
-// 123.8, 119.8, mixed 110.3, 107.7; 2048^2 FP32 313, 422).  2 rows, whose 4
+// and frame kernels: 512^2 FP64 72.5, 67.0, 600^2 94.8, 84.5, 300 x 1200 89.1,
+// 95.6; 900^2 FP32 93.3, 92.7, 1024^2 112.8, 112.2, mixed 102.9, 101.5).  2 rows, whose 4
 // wavefronts spread over the SIMDs, while one round of such tiles holds the
 // grid (128^2 FP64 25.3 us, with 7 rows 40.6); beyond, 7 rows in FP64 and 6 in
 // the float variants, which form less twice (512^2: 72.6 against 80.3 with 2
