@@ -940,7 +940,10 @@ hipError_t launch_fused_step(const e2d_params& p, const DevBuffers& b, const Ste
 }
 
 hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c, hipStream_t s) {
-  const TraceRange range("computeAndStoreFluxes");
+  // one kernel forms what the reference's three procedures do
+  const TraceRange prim("convertToPrimitives");
+  const TraceRange flux("computeAndStoreFluxes");
+  const TraceRange update("updateHydro");
   return with_precision(p.precision, [&](auto pol) {
     using P = decltype(pol);
     return p.implementation_version == E2D_IMPL_FLUX_STORE ? fused_step<P, 2>(p, b, c, s) : fused_step<P, 1>(p, b, c, s);
