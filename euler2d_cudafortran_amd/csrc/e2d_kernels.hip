@@ -689,10 +689,10 @@ void k_step_tile(const StepArgs<P> a) {
 // The materialised versions' step (STAGES 1 and 2) on the same march.  As six
 // and four kernels that passed q, slopes, face states and fluxes through HBM,
 // version 1 moved 3.5 GB and version 2 1.4 GB per 2048^2 FP64 step, at the rate
-// of a copy; here each stage is written once and read by nothing (1.67 GB and
-// 0.8 GB): 740 -> 340 us and 356 -> 220 us per step.  Version 1 is bound by its
-// writes; in FP64 it is held at 2 wavefronts per SIMD, since at 3 it spills
-// 60 B per lane (385 us).  Version 2 is bound by VALU issue, as the fused step.
+// of a copy; here each stage is written once and read by nothing (1.58 GB and
+// 0.79 GB): 756 -> 341 us and 356 -> 192 us per step.  Version 1 is bound by its
+// writes (4.6 TB/s); in FP64 it is held at 2 wavefronts per SIMD, since at 3 it
+// spills 60 B per lane (385 us).  Version 2 is bound by VALU issue, as the fused step.
 template <class P, int STAGES>
 constexpr int staged_waves() {
   return STAGES == 1 && sizeof(typename P::T) == 8 ? 2 : fused_waves<P>();

@@ -40,7 +40,7 @@ extern "C" {
 #define E2D_ERR_STATE (-4)    /* call not valid in the context's current state */
 
 /* implementation_version: cuf/m_HydroConstants.cuf:51-53 */
-#define E2D_IMPL_FUSED 0        /* one fused kernel per step (LDS-free register marching) */
+#define E2D_IMPL_FUSED 0        /* one fused kernel per step */
 #define E2D_IMPL_MATERIALISED 1 /* q, slopes, face states and fluxes stored in HBM */
 #define E2D_IMPL_FLUX_STORE 2   /* q and fluxes stored in HBM, slopes and face states in registers */
 
