@@ -86,12 +86,12 @@ __device__ __forceinline__ void store4(T* a, const Grid& g, int i, int j, const 
 }
 
 // primitives of cell (i, j) from the (boundary-filled) state, exactly as
-// k_adj_prim stores them
+// k_adj_prim stores them; returns cons_to_prim's result
 template <class P>
-__device__ __forceinline__ void prim_at(const AdjArgs<P>& a, int i, int j, typename P::T q[4]) {
+__device__ __forceinline__ typename P::T prim_at(const AdjArgs<P>& a, int i, int j, typename P::T q[4]) {
   typename P::T u[4];
   load4(a.u, a.g, i, j, u);
-  cons_to_prim<typename P::T, typename P::M>(a.h, u, q);
+  return cons_to_prim<typename P::T, typename P::M>(a.h, u, q);
 }
 
 // dt/dx and dt/dy as the forward step forms them (in the update type U)
@@ -293,8 +293,10 @@ __global__ __launch_bounds__(64 * kAdjWaves) E2D_ADJ_MARCH_ATTR void k_adj_march
   auto row = [&](int r) { return r < 0 ? 0 : (r > g.jsize - 1 ? g.jsize - 1 : r); };
 
   T qa[4], qb[4], qc[4];
-  prim_at(a, cl, row(ra - 2), qa);
-  prim_at(a, cl, row(ra - 1), qb);
+  const T pa = prim_at(a, cl, row(ra - 2), qa);
+  const T pb = prim_at(a, cl, row(ra - 1), qb);
+  // bits 0, 1, 2: row r+1, r, r-1 holds a cell that takes the limiter's long form
+  unsigned long_rows = (any_long_slope(pa) ? 2 : 0) + (any_long_slope(pb) ? 1 : 0);
   // row r-1, carried: slopes, trace sources and the bars of its xmin, xmax, ymin face states
   // (its primitives are qa)
   T pdx[4], pdy[4], ps[4], pbxm[4], pbxp[4], pbym[4];
@@ -310,7 +312,8 @@ __global__ __launch_bounds__(64 * kAdjWaves) E2D_ADJ_MARCH_ATTR void k_adj_march
 #pragma unroll
       for (int v = 0; v < 4; ++v) uc[v] = un[v];
       load4(a.u, g, cl, row(r + 2), un);
-      cons_to_prim<T, M>(a.h, uc, qc);
+      const T pc = cons_to_prim<T, M>(a.h, uc, qc);
+      long_rows = (long_rows << 1 | (any_long_slope(pc) ? 1 : 0)) & 7;
     }
     {
       const bool in = interior(g, ci, r);
@@ -323,7 +326,7 @@ __global__ __launch_bounds__(64 * kAdjWaves) E2D_ADJ_MARCH_ATTR void k_adj_march
       qxm[v] = from_left<true>(qb[v]);
       qxp[v] = from_right<true>(qb[v]);
     }
-    if (a.h.slope_type == 1)
+    if (a.h.slope_type == 1 && __builtin_expect(long_rows == 0, 1))
       cell_slopes<true>(a.h, qb, qxp, qxm, qc, qa, dqx, dqy);
     else
       cell_slopes(a.h, qb, qxp, qxm, qc, qa, dqx, dqy);
@@ -644,8 +647,10 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
   auto row = [&](int r) { return r < 0 ? 0 : (r > g.jsize - 1 ? g.jsize - 1 : r); };
 
   T qa[4], qb[4], qc[4];  // primitives of rows r-1, r, r+1
-  prim_at(a, cl, row(ra - 2), qa);
-  prim_at(a, cl, row(ra - 1), qb);
+  const T pa = prim_at(a, cl, row(ra - 2), qa);
+  const T pb = prim_at(a, cl, row(ra - 1), qb);
+  // bits 0, 1, 2: row r+1, r, r-1 holds a cell that takes the limiter's long form
+  unsigned long_rows = (any_long_slope(pa) ? 2 : 0) + (any_long_slope(pb) ? 1 : 0);
   // row r-1, carried: slopes, trace sources and the bars of its xmin, xmax, ymin face states
   T pdx[4], pdy[4], ps[4];
   // carried in LDS: partial sum of the last completed row, its plus part, the
@@ -681,7 +686,8 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
       for (int v = 0; v < 4; ++v) uc[v] = un[v];
       load4(a.u, g, cl, row(r + 2), un);
       energy(r + 1) = uc[1];
-      cons_to_prim<T, M>(a.h, uc, qc);
+      const T pc = cons_to_prim<T, M>(a.h, uc, qc);
+      long_rows = (long_rows << 1 | (any_long_slope(pc) ? 1 : 0)) & 7;
     }
     {
       const bool in = interior(g, ci, r);
@@ -696,7 +702,7 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
     }
     // (minmod's shorter form behind a uniform branch: 8 instructions for each of
     // 8 slopes instead of 15; 2048^2 FP64 us per adjoint step 556 -> 517)
-    if (a.h.slope_type == 1)
+    if (a.h.slope_type == 1 && __builtin_expect(long_rows == 0, 1))
       cell_slopes<true>(a.h, qb, qxp, qxm, qc, qa, dqx, dqy);
     else
       cell_slopes(a.h, qb, qxp, qxm, qc, qa, dqx, dqy);
@@ -901,6 +907,11 @@ constexpr int adj_tile_waves() {
 // states (what a wavefront keeps across a Riemann adjoint lies in LDS or is
 // formed again, as that alone takes 153 VGPRs in FP64)
 constexpr int adj_tile_lds_rows(int rows) { return (rows + 4) + (rows + 1) + 3 * rows; }
+// behind them a word per row of primitives (whether a cell of it takes the limiter's long form)
+template <class T>
+constexpr int adj_tile_lds_bytes(int rows) {
+  return adj_tile_lds_rows(rows) * 256 * static_cast<int>(sizeof(T)) + (rows + 4) * static_cast<int>(sizeof(int));
+}
 
 // cell (i, j) of the state with its ghost cells filled (corners as stored)
 template <class P>
@@ -949,6 +960,7 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
   T* const y_lds = q_lds + (R + 4) * 256;               // y-face k, between grid rows ra-1+k and ra+k
   T* const m_lds = y_lds + (R + 1) * 256;               // minus part of grid row ra + k, for the row below it
   T* const x_lds = m_lds + R * 256;                     // bars of the x-face states of grid row ra + k
+  int* const long_row = reinterpret_cast<int*>(x_lds + 2 * R * 256);  // as q_lds
   T* const qr = q_lds + (wave + 1) * 256 + lane;        // this lane's cell
   T* const xb = x_lds + (wave - 1) * 512 + lane;
 
@@ -960,7 +972,7 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
   // primitives
   double lam_r[4] = {0.0, 0.0, 0.0, 0.0};  // zero outside the interior
   if (has_row) {
-    auto load = [&](int j, T* to) {
+    auto load = [&](int j, T* to, int* to_long) {
       S raw[4];
       const Src s = filled_cell(a, cl, row(j), raw);
       if (s.ghost && cl == ci && row(j) == j) {
@@ -970,13 +982,13 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
       T u[4], q[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) u[v] = static_cast<T>(raw[v]);
-      cons_to_prim<T, M>(a.h, u, q);
+      *to_long = any_long_slope(cons_to_prim<T, M>(a.h, u, q));
 #pragma unroll
       for (int v = 0; v < 4; ++v) to[v * 64] = q[v];
     };
-    load(r, qr);
-    if (wave == 0) load(r - 1, qr - 256);
-    if (wave == nr + 1) load(r + 1, qr + 256);
+    load(r, qr, long_row + wave + 1);
+    if (wave == 0) load(r - 1, qr - 256, long_row);
+    if (wave == nr + 1) load(r + 1, qr + 256, long_row + wave + 2);
     if (interior(g, ci, r)) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) lam_r[v] = a.lam[at(g, ci, r, v)];
@@ -984,6 +996,10 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
   }
   __syncthreads();
 
+  bool short_slopes = false;
+  if (has_row)
+    short_slopes = a.h.slope_type == 1 &&
+                   __builtin_amdgcn_readfirstlane(long_row[wave] | long_row[wave + 1] | long_row[wave + 2]) == 0;
   // the row's slopes and trace sources, from LDS each time they are needed
   auto trace = [&](T q[4], T dqx[4], T dqy[4], T s[4]) {
     T xm[4], xp[4], ym[4], yp[4];
@@ -996,7 +1012,7 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
       ym[v] = qr[v * 64 - 256];
       yp[v] = qr[v * 64 + 256];
     }
-    if (a.h.slope_type == 1)
+    if (short_slopes)
       cell_slopes<true>(a.h, q, xp, xm, yp, ym, dqx, dqy);
     else
       cell_slopes(a.h, q, xp, xm, yp, ym, dqx, dqy);
@@ -1464,7 +1480,7 @@ hipError_t adjoint_step(const e2d_params& p, const DevBuffers& b, int buf, doubl
     a.nshort = 0;
     a.short_rows = 1;
     hipLaunchKernelGGL(k_adj_tile<P>, dim3(nstrips * a.nsegs), dim3(64 * (tile_rows + 2)),
-                       adj_tile_lds_rows(tile_rows) * 256 * sizeof(T), st, a);
+                       adj_tile_lds_bytes<T>(tile_rows), st, a);
     hipLaunchKernelGGL(k_adj_seam<P>, dim3((g.isize + 63) / 64, (2 + 2 * a.nsegs + 3) / 4), dim3(256), 0, st, a);
   } else if (passes == Passes::kSeparate) {
     hipLaunchKernelGGL(k_adj_prim<P>, dim3((g.isize + 63) / 64, (g.jsize + 3) / 4), dim3(256), 0, st, a);

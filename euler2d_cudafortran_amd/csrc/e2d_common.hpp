@@ -228,6 +228,13 @@ __device__ __forceinline__ T wave_max(T x) {
   return x;
 }
 
+// whether the cell of some lane takes the limiter's long form (uniform; 64 active
+// lanes), p being cons_to_prim's result
+template <class T>
+__device__ __forceinline__ bool any_long_slope(T p) {
+  return __builtin_amdgcn_ballot_w64(!slopes_short(p)) != 0;
+}
+
 __device__ __forceinline__ void atomic_max_nonneg(double* dst, double v) {
   // IEEE order of non-negative doubles equals the order of their bit patterns
   atomicMax(reinterpret_cast<unsigned long long*>(dst), static_cast<unsigned long long>(__double_as_longlong(v)));

@@ -235,19 +235,19 @@ __device__ __forceinline__ void source_cell(const StepArgs<P>& a, int ci, bool c
 }
 
 template <class P>
-__device__ __forceinline__ void prim_of(const Hydro<typename P::T>& h, const typename P::S raw[4],
-                                        typename P::T q[4], typename P::T& irho) {
+__device__ __forceinline__ typename P::T prim_of(const Hydro<typename P::T>& h, const typename P::S raw[4],
+                                                 typename P::T q[4], typename P::T& irho) {
   using T = typename P::T;
   T u[4];
 #pragma unroll
   for (int v = 0; v < 4; ++v) u[v] = static_cast<T>(raw[v]);
-  cons_to_prim<T, typename P::M>(h, u, q, irho);
+  return cons_to_prim<T, typename P::M>(h, u, q, irho);
 }
 template <class P>
-__device__ __forceinline__ void prim_of(const Hydro<typename P::T>& h, const typename P::S raw[4],
-                                        typename P::T q[4]) {
+__device__ __forceinline__ typename P::T prim_of(const Hydro<typename P::T>& h, const typename P::S raw[4],
+                                                 typename P::T q[4]) {
   typename P::T irho;
-  prim_of<P>(h, raw, q, irho);
+  return prim_of<P>(h, raw, q, irho);
 }
 
 // nothing in the step reads a stage array again: non-temporal
@@ -258,7 +258,7 @@ __device__ __forceinline__ void store_stage(X* a, const Grid& g, int i, int j, c
 }
 
 // kMinmod: instantiated for slope_type == 1 (the benchmark's minmod), whose
-// limiter then skips the products by st = 1 and the first-order select.
+// limiter has a short form (see cell_slopes) and needs no first-order select.
 // STAGES 1, 2: implementation versions 1 and 2, which store their stage arrays
 // on the way: q on every cell, slopes and face states on [1, size-2]^2, fx and
 // fy on [2, size-2]^2.  The input's ghost cells are filled, so every cell is
@@ -316,9 +316,12 @@ __device__ __forceinline__ void step_fused_body(const Args& a) {
   fetch_cell<P>(a, cl, j0 - 1, plain, raw_b);
   fetch_cell<P>(a, cl, j0, plain, raw_next);
   source_cell<P>(a, cl, col_ok, j0 - 2, plain, raw);
-  prim_of<P>(h, raw, qa);
+  const T pa = prim_of<P>(h, raw, qa);
   source_cell<P>(a, cl, col_ok, j0 - 1, plain, raw_b);
-  prim_of<P>(h, raw_b, qb, irb);
+  const T pb = prim_of<P>(h, raw_b, qb, irb);
+  // bits 0, 1, 2: row r+1, r, r-1 holds a cell that takes the limiter's long form
+  unsigned long_rows = 0;
+  if constexpr (kMinmod) long_rows = (any_long_slope(pa) ? 2 : 0) + (any_long_slope(pb) ? 1 : 0);
   if constexpr (STAGES != 0) {
     if (j0 == 2 && q_lane) {
       store_stage(a.q, g, ci, 0, qa);
@@ -390,7 +393,8 @@ __device__ __forceinline__ void step_fused_body(const Args& a) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) rows_in[(slot_w * 4 + v) * 64 + lane] = raw[v];
 #endif
-    prim_of<P>(h, raw, qc, irc);
+    const T pc = prim_of<P>(h, raw, qc, irc);
+    if constexpr (kMinmod) long_rows = (long_rows << 1 | (any_long_slope(pc) ? 1 : 0)) & 7;
     if constexpr (STAGES != 0) {
       // row r+1 in [j0, j1), and the topmost row with the last segment
       if (q_lane && (it < n_it - 2 || (it == n_it - 2 && j1 == g.ny + 2 + kMore))) store_stage(a.q, g, ci, r + 1, qc);
@@ -403,7 +407,10 @@ __device__ __forceinline__ void step_fused_body(const Args& a) {
       qxm[v] = from_left(qb[v]);
       qxp[v] = from_right(qb[v]);
     }
-    cell_slopes<kMinmod>(h, qb, qxp, qxm, qc, qa, dqx, dqy);
+    if (kMinmod && __builtin_expect(long_rows == 0, 1))
+      cell_slopes<true>(h, qb, qxp, qxm, qc, qa, dqx, dqy);
+    else
+      cell_slopes(h, qb, qxp, qxm, qc, qa, dqx, dqy);
     trace_sources<T, M>(h, qb, dqx, dqy, s, irb);
     if constexpr (STAGES == 1) {
       if (slope_lane && ((it >= 1 && it < n_it - 1) || (it == 0 && j0 == 2))) {
@@ -548,8 +555,13 @@ constexpr int tile_waves() {
   return sizeof(typename P::T) == 8 ? 6 : 8;
 }
 // rows of LDS (4 variables x 64 lanes of T) of a tile of R rows: primitives and
-// the lower states, then fluxes, of the y-faces
+// the lower states, then fluxes, of the y-faces; behind them a word per row of
+// primitives (whether a cell of it takes the limiter's long form)
 constexpr int tile_lds_rows(int rows) { return (rows + 4) + (rows + 1); }
+template <class T>
+constexpr int tile_lds_bytes(int rows) {
+  return tile_lds_rows(rows) * 256 * static_cast<int>(sizeof(T)) + (rows + 4) * static_cast<int>(sizeof(int));
+}
 
 template <class P, bool kMinmod>
 __global__ __launch_bounds__(64 * (kTileMaxRows + 2)) __attribute__((amdgpu_waves_per_eu(tile_waves<P>())))
@@ -580,6 +592,7 @@ void k_step_tile(const StepArgs<P> a) {
 
   T* const q_lds = reinterpret_cast<T*>(tile_mem);  // row k: grid row j0 - 2 + k
   T* const y_lds = q_lds + (R + 4) * 256;           // y-face k, between rows j0-1+k and j0+k
+  int* const long_row = reinterpret_cast<int*>(y_lds + (R + 1) * 256);  // as q_lds
 
   double invdt_cur = 0.0;
   if (a.dt_from_device) invdt_cur = invdt_part(a.scal, a.slot_cur);
@@ -591,15 +604,17 @@ void k_step_tile(const StepArgs<P> a) {
     fetch_cell<P>(a, cl, r, plain, raw);
     if (ends) fetch_cell<P>(a, cl, r2, plain, raw2);
     source_cell<P>(a, cl, col_ok, r, plain, raw);
-    prim_of<P>(h, raw, q, irho);
+    const T p = prim_of<P>(h, raw, q, irho);
 #pragma unroll
     for (int v = 0; v < 4; ++v) q_lds[((wave + 1) * 4 + v) * 64 + lane] = q[v];
+    if constexpr (kMinmod) long_row[wave + 1] = any_long_slope(p);
     if (ends) {
       T q2[4];
       source_cell<P>(a, cl, col_ok, r2, plain, raw2);
-      prim_of<P>(h, raw2, q2);
+      const T p2 = prim_of<P>(h, raw2, q2);
 #pragma unroll
       for (int v = 0; v < 4; ++v) q_lds[((r2 - j0 + 2) * 4 + v) * 64 + lane] = q2[v];
+      if constexpr (kMinmod) long_row[r2 - j0 + 2] = any_long_slope(p2);
     }
   }
   U dt;
@@ -619,8 +634,8 @@ void k_step_tile(const StepArgs<P> a) {
   S uold[4] = {S(0), S(0), S(0), S(0)};
   if (has_row) {
     T dqx[4], dqy[4], s[4];
-    {
-      const T* const qr = q_lds + (wave + 1) * 256;
+    const T* const qr = q_lds + (wave + 1) * 256;
+    auto slopes = [&](auto minmod) {
       T xm[4], xp[4], ym[4], yp[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -629,8 +644,13 @@ void k_step_tile(const StepArgs<P> a) {
         ym[v] = qr[v * 64 + lane - 256];
         yp[v] = qr[v * 64 + lane + 256];
       }
-      cell_slopes<kMinmod>(h, q, xp, xm, yp, ym, dqx, dqy);
-    }
+      cell_slopes<decltype(minmod)::value>(h, q, xp, xm, yp, ym, dqx, dqy);
+    };
+    if (kMinmod &&
+        __builtin_expect(__builtin_amdgcn_readfirstlane(long_row[wave] | long_row[wave + 1] | long_row[wave + 2]), 0) == 0)
+      slopes(std::true_type{});
+    else
+      slopes(std::false_type{});
     trace_sources<T, M>(h, q, dqx, dqy, s, irho);
     if (up_row) {
       T f[4];
@@ -880,7 +900,7 @@ static hipError_t launch_fused(Args& a, hipStream_t st) {
       a.nsegs = (a.g.ny + rows - 1) / rows;
       const int nstrips = (a.g.nx + kStripOut - 1) / kStripOut;
       hipLaunchKernelGGL((k_step_tile<P, kMinmod>), dim3(nstrips * a.nsegs), dim3(64 * (rows + 2)),
-                         tile_lds_rows(rows) * 256 * sizeof(typename P::T), st, a);
+                         tile_lds_bytes<typename P::T>(rows), st, a);
       return hipGetLastError();
     }
   }

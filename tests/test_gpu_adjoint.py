@@ -647,3 +647,30 @@ def test_adjoint_tiles_equal_the_march(gpu_lib, monkeypatch, nx, ny, bc, st, row
                 run.adjoint_step(0, dt, a, b)
                 got.append((run.field_download(b), run.download(0)))
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), prec
+
+
+@pytest.mark.parametrize("prec", [e2d.PREC_FP64, e2d.PREC_FP32, e2d.PREC_FP32_NATIVE, e2d.PREC_MIXED])
+def test_adjoint_beside_nonfinite_cells(gpu_lib, monkeypatch, prec):
+    """A state with NaN and infinite cells: the marching kernels and the tiles give the separate
+    passes' lam (these take the limiter as e2d_pointwise does), NaN where they have one."""
+    nx, ny = 130, 41
+    u = _smooth_state(nx, ny, 7)
+    u[nx // 2:, :, :2] *= 0.3
+    for k, (v, bad) in enumerate([(2, np.nan), (3, np.nan), (2, np.inf), (3, -np.inf), (1, np.inf), (0, np.inf)]):
+        u[6 + 20 * k, 4 + 9 * (k % 4), v] = bad
+        u[7 + 20 * k, 24 - 4 * (k % 4):26 - 4 * (k % 4), v] = bad
+    lam = np.where(_interior(nx, ny), np.random.default_rng(3).normal(size=u.shape), 0.0)
+    res = {}
+    for mode, tile in (("separate", 0), ("march", 0), ("fused", 0), ("fused", 2), ("fused", 7)):
+        monkeypatch.setenv("E2D_ADJOINT_PASSES", mode)
+        monkeypatch.setenv("E2D_ADJOINT_TILE_ROWS", str(tile))
+        with e2d.HydroRun(_params(nx, ny, precision=prec)) as run:
+            run.upload(0, u)
+            a, b = run.field_alloc(), run.field_alloc()
+            run.field_upload(a, lam)
+            run.adjoint_step(0, 1e-4, a, b)
+            res[mode, tile] = run.field_download(b)
+    want = res.pop(("separate", 0))
+    assert 0 < np.isnan(want).sum() < 0.1 * want.size
+    for k, got in res.items():
+        assert np.array_equal(got, want, equal_nan=True), (k, int((~((got == want) | np.isnan(want))).sum()))

@@ -457,3 +457,49 @@ def test_skipped_rates_never_set_dt(gpu_lib, monkeypatch, prec, nx, ny, tile):
                 res.append((run.download(0), run.download(1), run.invdt))
         assert res[0][2] == res[1][2] or (np.isnan(res[0][2]) and np.isnan(res[1][2])), kind
         assert _same(res[1][0], res[0][0]) and _same(res[1][1], res[0][1]), kind
+
+
+# ---------------------------------------------------------------------------
+# the limiter beside cells that are not finite
+
+def _nonfinite_state(nx, ny):
+    """A smooth flow with a jump, and NaN and infinite momenta, energies and densities in cells
+    apart from each other and two in neighbouring ones."""
+    x, y = np.meshgrid((np.arange(nx + 4) - 1.5) / nx, (np.arange(ny + 4) - 1.5) / ny, indexing="ij")
+    left = x + y < 1
+    rho = np.where(left, 1.0, 0.4) * (1 + 0.4 * np.sin(6 * x + 1) * np.cos(5 * y))
+    p = np.where(left, 1.0, 0.3) * (1 + 0.3 * np.cos(7 * x) * np.sin(4 * y))
+    vx, vy = 0.3 * np.sin(5 * x + 2 * y), 0.2 * np.cos(3 * x - 4 * y)
+    u = np.stack([rho, p / 0.4 + 0.5 * rho * (vx * vx + vy * vy), rho * vx, rho * vy], axis=-1)
+    inf, nan = np.inf, np.nan
+    for k, (v, bad) in enumerate([(2, nan), (3, nan), (2, inf), (3, -inf), (1, nan), (1, inf), (0, nan), (0, inf)]):
+        u[6 + 15 * k, 4 + 9 * (k % 4), v] = bad
+        u[7 + 15 * k, 24 - 4 * (k % 4):26 - 4 * (k % 4), v] = bad
+    return u
+
+
+@pytest.mark.parametrize("prec", [e2d.PREC_FP64, e2d.PREC_FP32, e2d.PREC_FP32_NATIVE, e2d.PREC_MIXED])
+def test_minmod_beside_nonfinite_cells(gpu_lib, monkeypatch, prec):
+    """The limiter's values beside NaN and infinite cells are the routine's: the slopes that version 1
+    stores against e2d_pointwise of its primitives, and version 0's state, marching and on tiles,
+    against version 1's, NaN where it has one."""
+    nx, ny, dt = 130, 41, 1e-4
+    u = _nonfinite_state(nx, ny)
+    with e2d.HydroRun(_params(nx, ny, 1, prec)) as run:
+        run.upload(0, u)
+        run.godunov_unsplit(0, dt)
+        q, dqx, dqy = (run.download_stage(n) for n in ("q", "dqx", "dqy"))
+        u2 = run.download(1)
+    assert 15 < (~np.isfinite(q)).sum() < 60
+    c, xp, xm, yp, ym = q[1:-1, 1:-1], q[2:, 1:-1], q[:-2, 1:-1], q[1:-1, 2:], q[1:-1, :-2]
+    dq = e2d.pointwise(_params(nx, ny, 1, prec), e2d.FN_SLOPE, np.concatenate([c, xp, xm, yp, ym], axis=-1).reshape(-1, 20))
+    dq = dq.reshape(c.shape[:2] + (8,))
+    assert _same(dqx[1:-1, 1:-1], dq[..., :4]), _diff_report(dqx[1:-1, 1:-1], dq[..., :4])
+    assert _same(dqy[1:-1, 1:-1], dq[..., 4:]), _diff_report(dqy[1:-1, 1:-1], dq[..., 4:])
+    for tile in (0, 3, 14):
+        monkeypatch.setenv("E2D_TILE_ROWS", str(tile))
+        with e2d.HydroRun(_params(nx, ny, 0, prec)) as run:
+            run.upload(0, u)
+            run.godunov_unsplit(0, dt)
+            got = run.download(1)
+        assert _same(got, u2), (tile, _diff_report(got, u2))
