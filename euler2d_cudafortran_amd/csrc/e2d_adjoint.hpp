@@ -144,7 +144,8 @@ E2D_HDI void cons_to_prim_adj(const Hydro<T>& h, const T u[4], const T qb[4], T 
 // The slope is dc where |dc| is the smallest part (ties and uniform states
 // included), else 0 where dl dr <= 0, else the smaller of dl and dr, whose sign
 // dc shares: whichever it is, the bar of that difference is ob itself, so two
-// selects place it and the middle one's bar is minus the sum of the other two.
+// selects place it and the middle one's bar is minus the sum of the other two,
+// which for dc is zero whatever ob is (an infinite or NaN one included).
 template <class T>
 E2D_HDI void limited_slope_adj(T st, T qm, T q0, T qp, T ob, T& qm_b,
                                T& q0_b, T& qp_b) {
@@ -161,7 +162,7 @@ E2D_HDI void limited_slope_adj(T st, T qm, T q0, T qp, T ob, T& qm_b,
   const T m = (centred || left) ? x : T(0.0);
   const T p = (centred || !left) ? x : T(0.0);
   qm_b -= m;
-  q0_b += m - p;
+  q0_b += centred ? T(0.0) : m - p;
   qp_b += p;
 }
 

@@ -55,13 +55,13 @@ def test_float_instantiation_against_double(report):
     assert p99 <= 1e-4, f"float vs double Riemann adjoint, 99th percentile {p99:.3e}"
 
 
-@pytest.mark.parametrize("dtype", ["double", "float"])
-def test_limiter_adjoint_branches(tmp_path, dtype):
+@pytest.mark.parametrize("dtype, bars", [("double", 2), ("float", 2), ("double-nonfinite", 3), ("float-nonfinite", 3)])
+def test_limiter_adjoint_branches(tmp_path, dtype, bars):
     # which difference the bar goes to, at ties and uniform states too: exact
     exe = tmp_path / "limiter_adjoint_check"
     subprocess.run([shutil.which("g++"), "-O2", "-std=c++17", "-ffp-contract=off", "-o", str(exe),
                     str(ROOT / "tests" / "limiter_adjoint_check.cpp")], check=True)
     out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
     m = re.search(rf"{dtype} n=(\d+) bad=(\d+)", out)
-    assert int(m.group(1)) == 2 * 13 ** 3 * 2
+    assert int(m.group(1)) == 2 * 13 ** 3 * bars
     assert int(m.group(2)) == 0
