@@ -153,15 +153,19 @@ int fill_slot(e2d_ctx* c, int slot, double v) {
   return E2D_OK;
 }
 
+// the maximum of a running-invDt slot's parts, `stride` doubles apart
+double largest_part(const double* parts, int stride) {
+  double m = parts[0];
+  for (int p = 1; p < e2d::kInvdtParts; ++p) m = m > parts[p * stride] ? m : parts[p * stride];
+  return m;
+}
+
 // value of running-invDt slot `slot` (the maximum of its parts); synchronous
 int read_slot(e2d_ctx* c, int slot, double* v) {
-  const double* parts = c->pinned;
   HIP_TRY(hipMemcpyAsync(c->pinned, c->b.scal + slot * e2d::kInvdtSlot, e2d::kInvdtSlot * sizeof(double),
                          hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  double m = parts[0];
-  for (int p = 1; p < e2d::kInvdtParts; ++p) m = m > parts[p * e2d::kInvdtStride] ? m : parts[p * e2d::kInvdtStride];
-  *v = m;
+  *v = largest_part(c->pinned, e2d::kInvdtStride);
   return E2D_OK;
 }
 
@@ -457,20 +461,24 @@ int e2d_compute_dt(e2d_ctx* c, int useU, double* dt) {
   if (!dt) return fail(E2D_ERR_ARG, "dt is NULL");
   if (int rc = pull_invdt(c)) return rc;
   const int buf = (useU == 0) ? 0 : 1;
-  // each block writes its maximum to host memory; their maximum by bit pattern
-  // is that of the device's atomic maxima (non-negative values)
+  // each block writes its maximum to host memory
   int nblocks = 0;
   HIP_TRY(timed(c, E2D_TIMER_DT,
                 [&] { return e2d::launch_block_invdt(c->p, c->b, buf, c->pinned, &nblocks, c->stream); }));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  uint64_t most = 0;
-  std::memcpy(&most, &c->invdt, sizeof(most));
+  // their maximum as the device's slots form it: block k folds into part k mod
+  // kInvdtParts by bit pattern (as invdt_fold, non-negative values), then the
+  // parts are compared, which loses a NaN part to the next one
+  uint64_t parts[e2d::kInvdtParts];
+  for (uint64_t& bits : parts) std::memcpy(&bits, &c->invdt, sizeof(bits));
   for (int k = 0; k < nblocks; ++k) {
     uint64_t bits;
     std::memcpy(&bits, c->pinned + k, sizeof(bits));
-    most = std::max(most, bits);
+    parts[k % e2d::kInvdtParts] = std::max(parts[k % e2d::kInvdtParts], bits);
   }
-  std::memcpy(&c->invdt, &most, sizeof(most));
+  double values[e2d::kInvdtParts];
+  std::memcpy(values, parts, sizeof(values));
+  c->invdt = largest_part(values, 1);
   *dt = dt_of(c->p, c->invdt);
   return E2D_OK;
 }

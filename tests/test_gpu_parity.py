@@ -503,3 +503,21 @@ def test_minmod_beside_nonfinite_cells(gpu_lib, monkeypatch, prec):
             run.godunov_unsplit(0, dt)
             got = run.download(1)
         assert _same(got, u2), (tile, _diff_report(got, u2))
+
+
+@pytest.mark.parametrize("prec", [e2d.PREC_FP64, e2d.PREC_FP32])
+def test_compute_dt_with_nan_cells(gpu_lib, prec):
+    """compute_dt of a uniform flow with a run of NaN cells, long enough that one block of the
+    reduction sees nothing else, is the uniform flow's, as the maximum over rates ignores NaN."""
+    nx = ny = 64
+    u = np.empty((nx + 4, ny + 4, 4))
+    u[...] = [1.0, 2.5, 0.3, -0.2]
+    bad = u.copy()
+    window = [(2 + t % (nx - 1), 2 + t // (nx - 1)) for t in range(5 * 256, 6 * 256)]  # the sixth block's cells
+    bad[tuple(np.array(window).T)] = np.nan
+    dts = []
+    for state in (u, bad):
+        with e2d.HydroRun(_params(nx, ny, 0, prec)) as run:
+            run.upload(0, state)
+            dts.append((run.compute_dt(0), run.invdt))
+    assert dts[0] == dts[1] and np.isfinite(dts[0][0])
