@@ -82,14 +82,17 @@ constexpr int kWavesPerBlock = E2D_WAVES_PER_BLOCK;
 // a sound speed: 4 divisions and a root of the update type).  The bound's terms
 // are those of cfl_rate; `slack` covers the cancellation of E / rho against the
 // kinetic energy, kRateMargin the roundings (about 20 of 2^-24 in the bound,
-// and cfl_rate's own in binary32).  A NaN or an infinity anywhere makes the
-// comparison false, and the rate is formed.  10 steps at 2048^2 FP64 1823 ->
+// and cfl_rate's own in binary32).  Where the energy is below 2^-60 or the
+// density above 2^60, which binary32 may hold as subnormal, zero or infinite,
+// the rate is formed; a density below binary32's normal range makes the bound
+// infinite or NaN, an infinite or NaN energy or momentum too, the comparison is
+// then false, and the rate is formed.  10 steps at 2048^2 FP64 1823 ->
 // 1778 us, 6 steps at 4096^2 mixed 2251 -> 2193, 3001 x 1537 fp32_native 641 -> 620
 // (with their sums).
 struct RateBound {
   float gg1, smallc2, smallr, inv_dx, inv_dy;  // gamma0 (gamma0 - 1), smallc^2
 };
-constexpr float kRateMargin = 1e-5f;
+constexpr float kRateMargin = 1e-5f, kRateLeast = 0x1p-60f;
 __device__ __forceinline__ float rate_limit_of(double invdt) {  // wave-uniform
   const float x = static_cast<float>(invdt) * (1.0f - kRateMargin);
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
@@ -99,11 +102,12 @@ __device__ __forceinline__ bool rate_below(const RateBound& b, const U u[4], flo
   const float ir = __builtin_amdgcn_rcpf(__builtin_fmaxf(static_cast<float>(static_cast<double>(u[0])), b.smallr));
   const float vx = __builtin_fabsf(static_cast<float>(static_cast<double>(u[2]))) * ir;
   const float vy = __builtin_fabsf(static_cast<float>(static_cast<double>(u[3]))) * ir;
-  const float e = static_cast<float>(static_cast<double>(u[1])) * ir;
+  const float energy = static_cast<float>(static_cast<double>(u[1]));
+  const float e = energy * ir;
   const float kin = 0.5f * (vx * vx + vy * vy);
   const float slack = 2e-6f * (__builtin_fabsf(e) + kin);
   const float c = __builtin_amdgcn_sqrtf(b.gg1 * (__builtin_fmaxf(e - kin, 0.0f) + slack) + b.smallc2);
-  return (c + vx) * b.inv_dx + (c + vy) * b.inv_dy < limit;
+  return (energy >= kRateLeast) & (ir >= kRateLeast) & ((c + vx) * b.inv_dx + (c + vy) * b.inv_dy < limit);
 }
 
 template <class P>

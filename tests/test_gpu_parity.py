@@ -521,3 +521,32 @@ def test_compute_dt_with_nan_cells(gpu_lib, prec):
             run.upload(0, state)
             dts.append((run.compute_dt(0), run.invdt))
     assert dts[0] == dts[1] and np.isfinite(dts[0][0])
+
+
+@pytest.mark.parametrize("tile", [0, 3])
+@pytest.mark.parametrize("scale, energy", [(1.0, 1.0), (1e39, 1e-4), (2e-38, 1e-6), (1e-40, 1.0)])
+def test_skipped_rates_past_the_range_of_binary32(gpu_lib, monkeypatch, scale, energy, tile):
+    """FP64 states whose densities and energies are infinite, subnormal or zero in binary32: a
+    blast wave, whose rates rise from step to step, gives the device-resident loop and the
+    host-driven one the same bits and running invDt."""
+    monkeypatch.setenv("E2D_TILE_ROWS", str(tile))
+    nx, ny = 64, 48
+    u = np.zeros((nx + 4, ny + 4, 4))
+    u[..., 0] = scale
+    u[..., 1] = scale * energy * 1e-3 / 0.4
+    u[24:40, 18:34, 1] = scale * energy * 10 / 0.4
+    res = []
+    for host in (True, False):
+        with e2d.HydroRun(_params(nx, ny, 0, e2d.PREC_FP64, smallr=1e-7 * scale)) as run:
+            run.upload(0, u)
+            start = run.compute_dt(0)
+            if host:
+                run.run_reference_loop(6)
+                run.compute_dt(0)
+            else:
+                run.make_boundaries(0)
+                run.run_steps(6)
+            res.append((run.download(0), run.download(1), run.invdt))
+            assert run.get_dt() < 0.8 * start
+    assert res[0][2] == res[1][2]
+    assert _same(res[1][0], res[0][0]) and _same(res[1][1], res[0][1])
