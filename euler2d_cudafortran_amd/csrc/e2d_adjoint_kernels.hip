@@ -907,11 +907,6 @@ constexpr int adj_tile_waves() {
 // states (what a wavefront keeps across a Riemann adjoint lies in LDS or is
 // formed again, as that alone takes 153 VGPRs in FP64)
 constexpr int adj_tile_lds_rows(int rows) { return (rows + 4) + (rows + 1) + 3 * rows; }
-// behind them a word per row of primitives (whether a cell of it takes the limiter's long form)
-template <class T>
-constexpr int adj_tile_lds_bytes(int rows) {
-  return adj_tile_lds_rows(rows) * 256 * static_cast<int>(sizeof(T)) + (rows + 4) * static_cast<int>(sizeof(int));
-}
 
 // cell (i, j) of the state with its ghost cells filled (corners as stored)
 template <class P>
@@ -960,7 +955,6 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
   T* const y_lds = q_lds + (R + 4) * 256;               // y-face k, between grid rows ra-1+k and ra+k
   T* const m_lds = y_lds + (R + 1) * 256;               // minus part of grid row ra + k, for the row below it
   T* const x_lds = m_lds + R * 256;                     // bars of the x-face states of grid row ra + k
-  int* const long_row = reinterpret_cast<int*>(x_lds + 2 * R * 256);  // as q_lds
   T* const qr = q_lds + (wave + 1) * 256 + lane;        // this lane's cell
   T* const xb = x_lds + (wave - 1) * 512 + lane;
 
@@ -972,7 +966,7 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
   // primitives
   double lam_r[4] = {0.0, 0.0, 0.0, 0.0};  // zero outside the interior
   if (has_row) {
-    auto load = [&](int j, T* to, int* to_long) {
+    auto load = [&](int j, T* to) {
       S raw[4];
       const Src s = filled_cell(a, cl, row(j), raw);
       if (s.ghost && cl == ci && row(j) == j) {
@@ -982,13 +976,13 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
       T u[4], q[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) u[v] = static_cast<T>(raw[v]);
-      *to_long = any_long_slope(cons_to_prim<T, M>(a.h, u, q));
+      cons_to_prim<T, M>(a.h, u, q);
 #pragma unroll
       for (int v = 0; v < 4; ++v) to[v * 64] = q[v];
     };
-    load(r, qr, long_row + wave + 1);
-    if (wave == 0) load(r - 1, qr - 256, long_row);
-    if (wave == nr + 1) load(r + 1, qr + 256, long_row + wave + 2);
+    load(r, qr);
+    if (wave == 0) load(r - 1, qr - 256);
+    if (wave == nr + 1) load(r + 1, qr + 256);
     if (interior(g, ci, r)) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) lam_r[v] = a.lam[at(g, ci, r, v)];
@@ -996,10 +990,7 @@ __attribute__((amdgpu_waves_per_eu(adj_tile_waves<typename P::T>()))) void k_adj
   }
   __syncthreads();
 
-  bool short_slopes = false;
-  if (has_row)
-    short_slopes = a.h.slope_type == 1 &&
-                   __builtin_amdgcn_readfirstlane(long_row[wave] | long_row[wave + 1] | long_row[wave + 2]) == 0;
+  const bool short_slopes = has_row && a.h.slope_type == 1 && !any_long_slope(sizes_of_rows(qr));
   // the row's slopes and trace sources, from LDS each time they are needed
   auto trace = [&](T q[4], T dqx[4], T dqy[4], T s[4]) {
     T xm[4], xp[4], ym[4], yp[4];
@@ -1480,7 +1471,7 @@ hipError_t adjoint_step(const e2d_params& p, const DevBuffers& b, int buf, doubl
     a.nshort = 0;
     a.short_rows = 1;
     hipLaunchKernelGGL(k_adj_tile<P>, dim3(nstrips * a.nsegs), dim3(64 * (tile_rows + 2)),
-                       adj_tile_lds_bytes<T>(tile_rows), st, a);
+                       adj_tile_lds_rows(tile_rows) * 256 * sizeof(T), st, a);
     hipLaunchKernelGGL(k_adj_seam<P>, dim3((g.isize + 63) / 64, (2 + 2 * a.nsegs + 3) / 4), dim3(256), 0, st, a);
   } else if (passes == Passes::kSeparate) {
     hipLaunchKernelGGL(k_adj_prim<P>, dim3((g.isize + 63) / 64, (g.jsize + 3) / 4), dim3(256), 0, st, a);

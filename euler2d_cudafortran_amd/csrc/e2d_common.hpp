@@ -229,10 +229,19 @@ __device__ __forceinline__ T wave_max(T x) {
 }
 
 // whether the cell of some lane takes the limiter's long form (uniform; 64 active
-// lanes), p being cons_to_prim's result
+// lanes); size as for slopes_short
 template <class T>
-__device__ __forceinline__ bool any_long_slope(T p) {
-  return __builtin_amdgcn_ballot_w64(!slopes_short(p)) != 0;
+__device__ __forceinline__ bool any_long_slope(T size) {
+  return __builtin_amdgcn_ballot_w64(!slopes_short(size)) != 0;
+}
+// such a size of a lane's cell and the cells below and above it, of primitives in
+// LDS (rows of 4 variables x 64 lanes; c: the cell's variable 0)
+template <class T>
+__device__ __forceinline__ T sizes_of_rows(const T* c) {
+  T size = T(0);
+#pragma unroll
+  for (int k = -256; k <= 256; k += 256) size += fabs_(c[k + 128]) + fabs_(c[k + 192]) + c[k + 64];
+  return size;
 }
 
 __device__ __forceinline__ void atomic_max_nonneg(double* dst, double v) {

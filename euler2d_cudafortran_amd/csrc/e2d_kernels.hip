@@ -559,13 +559,8 @@ constexpr int tile_waves() {
   return sizeof(typename P::T) == 8 ? 6 : 8;
 }
 // rows of LDS (4 variables x 64 lanes of T) of a tile of R rows: primitives and
-// the lower states, then fluxes, of the y-faces; behind them a word per row of
-// primitives (whether a cell of it takes the limiter's long form)
+// the lower states, then fluxes, of the y-faces
 constexpr int tile_lds_rows(int rows) { return (rows + 4) + (rows + 1); }
-template <class T>
-constexpr int tile_lds_bytes(int rows) {
-  return tile_lds_rows(rows) * 256 * static_cast<int>(sizeof(T)) + (rows + 4) * static_cast<int>(sizeof(int));
-}
 
 template <class P, bool kMinmod>
 __global__ __launch_bounds__(64 * (kTileMaxRows + 2)) __attribute__((amdgpu_waves_per_eu(tile_waves<P>())))
@@ -596,7 +591,6 @@ void k_step_tile(const StepArgs<P> a) {
 
   T* const q_lds = reinterpret_cast<T*>(tile_mem);  // row k: grid row j0 - 2 + k
   T* const y_lds = q_lds + (R + 4) * 256;           // y-face k, between rows j0-1+k and j0+k
-  int* const long_row = reinterpret_cast<int*>(y_lds + (R + 1) * 256);  // as q_lds
 
   double invdt_cur = 0.0;
   if (a.dt_from_device) invdt_cur = invdt_part(a.scal, a.slot_cur);
@@ -608,17 +602,15 @@ void k_step_tile(const StepArgs<P> a) {
     fetch_cell<P>(a, cl, r, plain, raw);
     if (ends) fetch_cell<P>(a, cl, r2, plain, raw2);
     source_cell<P>(a, cl, col_ok, r, plain, raw);
-    const T p = prim_of<P>(h, raw, q, irho);
+    prim_of<P>(h, raw, q, irho);
 #pragma unroll
     for (int v = 0; v < 4; ++v) q_lds[((wave + 1) * 4 + v) * 64 + lane] = q[v];
-    if constexpr (kMinmod) long_row[wave + 1] = any_long_slope(p);
     if (ends) {
       T q2[4];
       source_cell<P>(a, cl, col_ok, r2, plain, raw2);
-      const T p2 = prim_of<P>(h, raw2, q2);
+      prim_of<P>(h, raw2, q2);
 #pragma unroll
       for (int v = 0; v < 4; ++v) q_lds[((r2 - j0 + 2) * 4 + v) * 64 + lane] = q2[v];
-      if constexpr (kMinmod) long_row[r2 - j0 + 2] = any_long_slope(p2);
     }
   }
   U dt;
@@ -650,8 +642,7 @@ void k_step_tile(const StepArgs<P> a) {
       }
       cell_slopes<decltype(minmod)::value>(h, q, xp, xm, yp, ym, dqx, dqy);
     };
-    if (kMinmod &&
-        __builtin_expect(__builtin_amdgcn_readfirstlane(long_row[wave] | long_row[wave + 1] | long_row[wave + 2]), 0) == 0)
+    if (kMinmod && __builtin_expect(!any_long_slope(sizes_of_rows(qr + lane)), 1))
       slopes(std::true_type{});
     else
       slopes(std::false_type{});
@@ -904,7 +895,7 @@ static hipError_t launch_fused(Args& a, hipStream_t st) {
       a.nsegs = (a.g.ny + rows - 1) / rows;
       const int nstrips = (a.g.nx + kStripOut - 1) / kStripOut;
       hipLaunchKernelGGL((k_step_tile<P, kMinmod>), dim3(nstrips * a.nsegs), dim3(64 * (rows + 2)),
-                         tile_lds_bytes<typename P::T>(rows), st, a);
+                         tile_lds_rows(rows) * 256 * sizeof(typename P::T), st, a);
       return hipGetLastError();
     }
   }

@@ -345,7 +345,7 @@ E2D_HDI T cfl_rate(const Hydro<T>& h, const T u[4]) {
 // minimum and not of the other, and its sign says nothing), so callers take the
 // long form wherever slopes_short is false for one of the cells: a comparison a
 // cell and a uniform branch (2048^2 us per step without and with them: FP64
-// 167.0, 167.3, FP32 90.9, 91.9; 128^2 FP64 8.23, 8.45; in its place the long
+// 167.0, 167.3, FP32 90.9, 91.9; 128^2 FP64 8.24, 8.43; in its place the long
 // form everywhere is 2-3%).
 template <class T>
 E2D_HDI T with_sign_of(T magnitude, T sign) { return __builtin_copysign(magnitude, sign); }
@@ -370,13 +370,15 @@ E2D_HDI T limited_slope(T st, T qm, T q0, T qp) {
   return limited_slope_st<false>(st, qm, q0, qp);
 }
 
-// Whether a cell's differences to others like it are finite, from its pressure
-// before the floor (cons_to_prim's result), which holds rho (E / rho - the
-// kinetic energy): where that is finite the velocities are below the root of
-// the type's limit, and densities and pressures are positive.
+// Whether a cell's differences to others like it are finite, from its size: the
+// sum of its pressure and its velocities' magnitudes, or its pressure before the
+// floor (cons_to_prim's result), which holds rho (E / rho - the kinetic energy),
+// so that where it is finite the velocities are below the root of the type's
+// limit.  Densities and pressures are positive, and where a density is infinite
+// the pressure is infinite or NaN.
 template <class T>
-E2D_HDI bool slopes_short(T p) {
-  return fabs_(p) < (sizeof(T) == 8 ? T(0x1p1000) : T(0x1p100f));
+E2D_HDI bool slopes_short(T size) {
+  return fabs_(size) < (sizeof(T) == 8 ? T(0x1p1000) : T(0x1p100f));
 }
 
 // Slopes of a cell in both directions.  slope_type 0 and values other than
