@@ -821,7 +821,10 @@ int e2d_adjoint_rollout(e2d_ctx* c, int nStep0, int nsteps, const double* dts, i
   r.start_in_buffer = true;  // a recording has been compared with it
   if (int rc = r.reverse(0, nsteps, 0)) return rc;
   if (r.cur == 1) HIP_TRY(hipMemcpyAsync(lam_0, c->lam_tmp, field_bytes(c), hipMemcpyDeviceToDevice, c->stream));
-  if (!r.start_in_buffer)
+  // the starting state with its ghost cells filled, as the step from it leaves it
+  if (r.start_in_buffer)
+    HIP_TRY(e2d::launch_boundaries(c->p, c->b, nStep0 % 2, c->stream));
+  else
     HIP_TRY(hipMemcpyAsync(r.buffer_of(0), c->snapshots[0], state_bytes(c), hipMemcpyDeviceToDevice, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   if (n_forward) *n_forward = r.nfwd;

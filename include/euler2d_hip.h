@@ -264,8 +264,8 @@ int e2d_adjoint_step(e2d_ctx *ctx, int buf, double dt, const double *d_lam_in, d
  * Binomial checkpointing (Griewank and Walther's revolve schedule: the least
  * number of forward steps for nsnap kept states) keeps at most nsnap state
  * snapshots in device memory; *n_forward returns the number of forward steps
- * recomputed.  On return the starting state is back in its
- * buffer. */
+ * recomputed.  On return the starting state is back in its buffer, its
+ * non-corner ghost cells filled; the other buffer holds scratch. */
 int e2d_adjoint_rollout(e2d_ctx *ctx, int nStep0, int nsteps, const double *h_dts, int nsnap,
                         const double *d_lam_n, double *d_lam_0, int64_t *n_forward);
 

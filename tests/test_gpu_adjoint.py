@@ -674,3 +674,30 @@ def test_adjoint_beside_nonfinite_cells(gpu_lib, monkeypatch, prec):
     assert 0 < np.isnan(want).sum() < 0.1 * want.size
     for k, got in res.items():
         assert np.array_equal(got, want, equal_nan=True), (k, int((~((got == want) | np.isnan(want))).sum()))
+
+
+@pytest.mark.parametrize("n0, bc", [(0, (1, 2, 3, 1)), (1, (3, 3, 1, 2))])
+def test_rollout_leaves_the_start_with_filled_ghosts(gpu_lib, n0, bc):
+    """After an adjoint rollout, recorded or not, the buffer it started from holds the starting state
+    with its ghost cells filled and its corners as they were, whatever the numbers of steps and
+    snapshots, and whatever the ghost cells held."""
+    nx, ny = 40, 30
+    kw = dict(zip(("boundary_type_xmin", "boundary_type_xmax", "boundary_type_ymin", "boundary_type_ymax"), bc))
+    u = _smooth_state(nx, ny, 7)
+    u[~_interior(nx, ny)] *= 0.5
+    with e2d.HydroRun(_params(nx, ny, **kw)) as run:
+        run.upload(n0, u)
+        run.make_boundaries(n0)
+        want = run.download(n0)
+        assert not np.array_equal(u, want)
+        a, b = run.field_alloc(), run.field_alloc()
+        run.field_upload(a, np.where(_interior(nx, ny), 1.0, 0.0))
+        for nsteps in (1, 2, 3, 4, 7):
+            for nsnap in (1, 2, 3, 5):
+                for record in (False, True):
+                    run.upload(n0, u)
+                    if record:
+                        run.rollout_forward(n0, np.full(nsteps, 2e-3), nsnap)
+                        run.upload(n0, u)
+                    run.adjoint_rollout(n0, np.full(nsteps, 2e-3), nsnap, a, b)
+                    assert np.array_equal(run.download(n0), want), (nsteps, nsnap, record)
