@@ -1514,7 +1514,7 @@ size_t adjoint_scratch_elem_bytes(int precision) {
 
 hipError_t launch_adjoint_step(const e2d_params& p, const DevBuffers& b, int buf, double dt, const double* lam_in,
                                double* lam_out, const AdjointScratch& s, hipStream_t st) {
-  return with_precision(p.precision, [&](auto pol) {
+  return with_arithmetic(p, [&](auto pol) {
     return adjoint_step<decltype(pol)>(p, b, buf, dt, lam_in, lam_out, s, st);
   });
 }

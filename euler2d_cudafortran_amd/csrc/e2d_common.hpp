@@ -29,6 +29,7 @@ struct Prec {
 };
 using P64 = Prec<double, double, double, RangedMath, RangedMath>;
 using P32 = Prec<float, float, float, RangedMath, RangedMath>;
+using P32Low = Prec<float, float, float, LowFloorMath, LowFloorMath>;
 // FP32 state; FP32 flux arithmetic with the native reciprocal and square
 // root; the update added in FP64 and rounded to the FP32 state
 using PNative = Prec<float, float, double, FastMath, RangedMath>;
@@ -46,6 +47,21 @@ inline auto with_precision(int precision, F&& f) {
     case E2D_PREC_FP32_NATIVE: return f(PNative{});
     default: return f(PMix{});
   }
+}
+
+// Whether the floors of smallr and smallc allow a radicand below 2^-102: of the
+// Riemann solver (gamma0 smallr^2 smallp (1 - gamma6) = smallr^2 smallc^2
+// (1 - gamma6) at least) or of a sound speed (smallc^2).  1e-7 for both gives 2^-96.
+inline bool low_floors(const e2d_params& p) {
+  const double gamma6 = (p.gamma0 + 1.0) / (2.0 * p.gamma0);
+  const double sound = p.smallc * p.smallc, riemann = p.smallr * p.smallr * sound * (1.0 - gamma6);
+  return !(riemann >= 0x1p-102) || !(sound >= 0x1p-102);
+}
+// with_precision for kernels that take quotients and roots
+template <class F>
+inline auto with_arithmetic(const e2d_params& p, F&& f) {
+  if (p.precision == E2D_PREC_FP32 && low_floors(p)) return f(P32Low{});
+  return with_precision(p.precision, f);
 }
 
 // Derived parameters in precision T, as initHydroParameters computes them

@@ -519,7 +519,7 @@ template <class P>
 constexpr int fused_waves() {
   if constexpr (sizeof(typename P::T) > 8) return 1;
   else if constexpr (sizeof(typename P::T) == 8) return 3;
-  else if constexpr (std::is_same<typename P::M, RangedMath>::value) return 5;
+  else if constexpr (!std::is_same<typename P::M, FastMath>::value) return 5;
   else return 4;
 }
 
@@ -951,7 +951,7 @@ static hipError_t fused_step(const e2d_params& p, const DevBuffers& b, const Ste
 }
 
 hipError_t launch_fused_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c, hipStream_t s) {
-  return with_precision(p.precision, [&](auto pol) { return fused_step<decltype(pol), 0>(p, b, c, s); });
+  return with_arithmetic(p, [&](auto pol) { return fused_step<decltype(pol), 0>(p, b, c, s); });
 }
 
 hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, const StepCfg& c, hipStream_t s) {
@@ -959,7 +959,7 @@ hipError_t launch_materialised_step(const e2d_params& p, const DevBuffers& b, co
   const TraceRange prim("convertToPrimitives");
   const TraceRange flux("computeAndStoreFluxes");
   const TraceRange update("updateHydro");
-  return with_precision(p.precision, [&](auto pol) {
+  return with_arithmetic(p, [&](auto pol) {
     using P = decltype(pol);
     return p.implementation_version == E2D_IMPL_FLUX_STORE ? fused_step<P, 2>(p, b, c, s) : fused_step<P, 1>(p, b, c, s);
   });
@@ -1134,14 +1134,13 @@ static hipError_t max_invdt(const e2d_params& p, const DevBuffers& b, int buf, i
 }
 
 hipError_t launch_max_invdt(const e2d_params& p, const DevBuffers& b, int buf, int slot, hipStream_t s) {
-  return with_precision(p.precision,
-                        [&](auto pol) { return max_invdt<decltype(pol)>(p, b, buf, slot, nullptr, nullptr, s); });
+  return with_arithmetic(p,
+                         [&](auto pol) { return max_invdt<decltype(pol)>(p, b, buf, slot, nullptr, nullptr, s); });
 }
 
 hipError_t launch_block_invdt(const e2d_params& p, const DevBuffers& b, int buf, double* out, int* nblocks,
                               hipStream_t s) {
-  return with_precision(p.precision,
-                        [&](auto pol) { return max_invdt<decltype(pol)>(p, b, buf, 0, out, nblocks, s); });
+  return with_arithmetic(p, [&](auto pol) { return max_invdt<decltype(pol)>(p, b, buf, 0, out, nblocks, s); });
 }
 
 __global__ void k_fill(double* dst, int n, double v) {
@@ -1510,7 +1509,7 @@ __global__ __launch_bounds__(256) void k_pointwise(const Hydro<typename P::T> h,
 
 hipError_t launch_pointwise(const e2d_params& p, int func, int n, const double* d_x, double* d_y, hipStream_t s) {
   const dim3 grid((n + 255) / 256);
-  with_precision(p.precision, [&](auto pol) {
+  with_arithmetic(p, [&](auto pol) {
     using P = decltype(pol);
     hipLaunchKernelGGL(k_pointwise<P>, grid, dim3(256), 0, s, make_hydro<typename P::T>(p), func, n, d_x, d_y);
     return 0;

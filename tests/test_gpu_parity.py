@@ -550,3 +550,18 @@ def test_skipped_rates_past_the_range_of_binary32(gpu_lib, monkeypatch, scale, e
             assert run.get_dt() < 0.8 * start
     assert res[0][2] == res[1][2]
     assert _same(res[1][0], res[0][0]) and _same(res[1][1], res[0][1])
+
+
+@pytest.mark.parametrize("prec", [e2d.PREC_FP64, e2d.PREC_FP32])
+def test_cold_cells_set_dt_below_the_range_of_binary32(gpu_lib, prec):
+    """A sound-speed floor whose square is subnormal in binary32: a fast cold stream, its pressure at
+    the floor, still sets dt, c being nothing beside |u| (the oracle's formula with c = 0)."""
+    nx, ny = 64, 48
+    u = np.zeros((nx + 4, ny + 4, 4))
+    u[...] = [1.0, 2.5, 0.0, 0.0]
+    u[20:30, 10:40] = [1.0, 128.0, 16.0, 0.0]  # E is the kinetic energy
+    for smallc in (1e-7, 1e-18, 1e-20, 1e-22):
+        with e2d.HydroRun(_params(nx, ny, 0, prec, smallc=smallc)) as run:
+            run.upload(0, u)
+            dt = run.compute_dt(0)
+        assert abs(dt * 16 * nx / 0.8 - 1) < 1e-6, (smallc, dt)
