@@ -1297,36 +1297,44 @@ hipError_t launch_zero_state(const e2d_params& p, const DevBuffers& b, int buf, 
 // deterministic FP64 sums over the interior: block k reduces rows k, k+B, ...
 // in a fixed order, then one block adds the partials in block order.  Bound by
 // the memory's latency: a thread adds its values one by one, so it loads
-// kSumAhead of them (times 4 variables) before it adds the first (960
-// wavefronts with 4 loads in flight each read 134 MB in 34 us and 537 MB in
-// 186; with 32 in flight, 22 and 119), and the partials pass through LDS (added
-// from memory one by one they took 30 us, now 4).  The order of the additions
-// is the same.
+// kSumAhead of them (times 4 variables) before it adds the first, of one row or
+// of several (960 wavefronts with 4 loads in flight each read 134 MB in 34 us and
+// 537 MB in 186; with 32 in flight, 22 and 119), and the partials pass through
+// LDS (added from memory one by one they took 30 us, now 4).  The order of the
+// additions is the same.
 constexpr int kSumAhead = 8;
 
 template <class S>
 __global__ __launch_bounds__(256) void k_sums_partial(const Grid g, const S* __restrict__ u, double* partial) {
   __shared__ double red[4][256];
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int j = 2 + blockIdx.x; j <= g.ny + 1; j += gridDim.x)
-    for (int i0 = 2; i0 <= g.nx + 1; i0 += kSumAhead * 256) {
-      S x[kSumAhead][4];
+  const int tid = static_cast<int>(threadIdx.x);
+  int j = 2 + static_cast<int>(blockIdx.x), i0 = 0;  // the row and the column (from the first interior one) of thread 0
+  while (j <= g.ny + 1) {
+    S x[kSumAhead][4];
 #pragma unroll
-      for (int k = 0; k < kSumAhead; ++k) {
-        const int i = i0 + k * 256 + static_cast<int>(threadIdx.x);
+    for (int k = 0; k < kSumAhead; ++k) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) x[k][v] = S(0);
-        if (i0 + k * 256 <= g.nx + 1 && i <= g.nx + 1) {  // the first test is uniform
+      for (int v = 0; v < 4; ++v) x[k][v] = S(0);
+      if (j <= g.ny + 1) {  // uniform, as the address of the row
+        const S* const row = u + static_cast<int64_t>(j) * g.pitch + (2 + i0);
+        if (i0 + tid < g.nx) {
 #pragma unroll
-          for (int v = 0; v < 4; ++v) x[k][v] = u[at(g, i, j, v)];
+          for (int v = 0; v < 4; ++v) x[k][v] = row[v * g.plane + tid];
+        }
+        i0 += 256;
+        if (i0 >= g.nx) {
+          i0 = 0;
+          j += static_cast<int>(gridDim.x);
         }
       }
-      // a zero in the place of a column past the last leaves a sum as it is (no sum is -0)
-#pragma unroll
-      for (int k = 0; k < kSumAhead; ++k)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[v] += static_cast<double>(x[k][v]);
     }
+    // a zero in the place of a column past the last leaves a sum as it is (no sum is -0)
+#pragma unroll
+    for (int k = 0; k < kSumAhead; ++k)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[v] += static_cast<double>(x[k][v]);
+  }
 #pragma unroll
   for (int v = 0; v < 4; ++v) red[v][threadIdx.x] = acc[v];
   __syncthreads();

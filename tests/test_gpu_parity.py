@@ -565,3 +565,27 @@ def test_cold_cells_set_dt_below_the_range_of_binary32(gpu_lib, prec):
             run.upload(0, u)
             dt = run.compute_dt(0)
         assert abs(dt * 16 * nx / 0.8 - 1) < 1e-6, (smallc, dt)
+
+
+@pytest.mark.parametrize("prec", [e2d.PREC_FP64, e2d.PREC_FP32])
+@pytest.mark.parametrize("nx, ny", [(4, 4), (4, 5000), (255, 700), (256, 241), (257, 9), (2049, 12), (5000, 5)])
+def test_sums_keep_their_order(gpu_lib, prec, nx, ny):
+    """Narrow and wide rows, fewer and more rows than blocks: the sums are those of the stated order,
+    bit for bit: 240 blocks over rows, 256 threads over columns, halves of the threads, then the
+    blocks one after the other."""
+    u = np.random.default_rng(nx + ny).uniform(0.1, 2, (nx + 4, ny + 4, 4))
+    with e2d.HydroRun(_params(nx, ny, 0, prec)) as run:
+        run.upload(0, u)
+        got = run.sums(0)
+        inner = run.download(0)[2:-2, 2:-2]
+    acc = np.zeros((240, 256, 4))
+    for j in range(ny):
+        for i in range(0, nx, 256):
+            part = inner[i:i + 256, j]
+            acc[j % 240, :len(part)] += part
+    for w in (128, 64, 32, 16, 8, 4, 2, 1):
+        acc[:, :w] += acc[:, w:2 * w]
+    want = np.zeros(4)
+    for b in range(240):
+        want += acc[b, 0]
+    assert np.array_equal(got, want)
