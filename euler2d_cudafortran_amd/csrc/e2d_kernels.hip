@@ -411,10 +411,10 @@ __device__ __forceinline__ void step_fused_body(const Args& a) {
       qxm[v] = from_left(qb[v]);
       qxp[v] = from_right(qb[v]);
     }
-    if (kMinmod && __builtin_expect(long_rows == 0, 1))
-      cell_slopes<true>(h, qb, qxp, qxm, qc, qa, dqx, dqy);
+    if (kMinmod && __builtin_expect(long_rows != 0, 0))
+      cell_slopes<kMinmod, true>(h, qb, qxp, qxm, qc, qa, dqx, dqy);
     else
-      cell_slopes(h, qb, qxp, qxm, qc, qa, dqx, dqy);
+      cell_slopes<kMinmod>(h, qb, qxp, qxm, qc, qa, dqx, dqy);
     trace_sources<T, M>(h, qb, dqx, dqy, s, irb);
     if constexpr (STAGES == 1) {
       if (slope_lane && ((it >= 1 && it < n_it - 1) || (it == 0 && j0 == 2))) {
@@ -631,7 +631,7 @@ void k_step_tile(const StepArgs<P> a) {
   if (has_row) {
     T dqx[4], dqy[4], s[4];
     const T* const qr = q_lds + (wave + 1) * 256;
-    auto slopes = [&](auto minmod) {
+    auto slopes = [&](auto take_long) {
       T xm[4], xp[4], ym[4], yp[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -640,9 +640,9 @@ void k_step_tile(const StepArgs<P> a) {
         ym[v] = qr[v * 64 + lane - 256];
         yp[v] = qr[v * 64 + lane + 256];
       }
-      cell_slopes<decltype(minmod)::value>(h, q, xp, xm, yp, ym, dqx, dqy);
+      cell_slopes<kMinmod, decltype(take_long)::value>(h, q, xp, xm, yp, ym, dqx, dqy);
     };
-    if (kMinmod && __builtin_expect(!any_long_slope(sizes_of_rows(qr + lane)), 1))
+    if (kMinmod && __builtin_expect(any_long_slope(sizes_of_rows(qr + lane)), 0))
       slopes(std::true_type{});
     else
       slopes(std::false_type{});

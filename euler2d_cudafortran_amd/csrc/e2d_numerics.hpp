@@ -383,7 +383,7 @@ E2D_HDI T cfl_rate(const Hydro<T>& h, const T u[4]) {
 // minimum and not of the other, and its sign says nothing), so callers take the
 // long form wherever slopes_short is false for one of the cells: a comparison a
 // cell and a uniform branch (2048^2 us per step without and with them: FP64
-// 167.0, 167.3, FP32 90.9, 91.9; 128^2 FP64 8.24, 8.43; in its place the long
+// 173.6, 174.7, FP32 93.9, 94.5; 128^2 FP64 8.22, 8.27; in its place the long
 // form everywhere is 2-3%).
 template <class T>
 E2D_HDI T with_sign_of(T magnitude, T sign) { return __builtin_copysign(magnitude, sign); }
@@ -421,17 +421,18 @@ E2D_HDI bool slopes_short(T size) {
 
 // Slopes of a cell in both directions.  slope_type 0 and values other than
 // 1/2 give zero slopes (first order), m_utils.f90:289-337.  kMinmod: the
-// caller knows slope_type == 1 and slopes_short of the five cells, so the
-// limiter takes its short form and skips the first-order select.
-template <bool kMinmod = false, class T>
+// caller knows slope_type == 1, so the limiter skips the products by st = 1 and
+// the first-order select, and, unless kLong, slopes_short of the five cells, so
+// that it takes its short form.
+template <bool kMinmod = false, bool kLong = false, class T>
 E2D_HDI void cell_slopes(const Hydro<T>& h, const T q[4], const T qxp[4],
                                             const T qxm[4], const T qyp[4], const T qym[4],
                                             T dqx[4], T dqy[4]) {
   if (kMinmod) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      dqx[v] = limited_slope_st<true>(T(1), qxm[v], q[v], qxp[v]);
-      dqy[v] = limited_slope_st<true>(T(1), qym[v], q[v], qyp[v]);
+      dqx[v] = limited_slope_st<!kLong>(T(1), qxm[v], q[v], qxp[v]);
+      dqy[v] = limited_slope_st<!kLong>(T(1), qym[v], q[v], qyp[v]);
     }
     return;
   }
