@@ -1428,6 +1428,7 @@ int plan_adjoint_tile(const Grid& g, size_t elem) {
                            "E2D_ADJOINT_LONG_PCT", "E2D_ADJOINT_CHUNK"})
     if (getenv(name)) return 0;
   const int64_t strips = (g.isize + kFusedStripOut - 1) / kFusedStripOut;
+  if (strips * g.ny > 100 * cus) return 0;
   const int64_t tiles = strips * ((g.jsize - 2 + 1) / 2);
   const int64_t round = cus * (elem == 8 ? 4 * adj_tile_waves<double>() : 4 * adj_tile_waves<float>()) / 4;
   if (tiles <= round) return 2;

@@ -851,13 +851,19 @@ static int plan_segments(StepArgs<P>& a, int ncols, int ny, int wps, int residen
 
 // Rows per tile, or 0 for the marching kernel.  Tiles up to 2,700 cells per
 // compute unit in FP64 and 2,400 in the float variants (about 830^2 and 780^2),
-// where the two cross.  us per step, march against tiles: 640^2 FP64 36.6,
-// 30.5; 800^2 48.1, 45.7; 900^2 53.7, 57.4; 1000 x 610 FP32 27.2, 23.5; 800^2
-// 27.6, 29.7; 640^2 fp32_native 20.8, 16.5; 800^2 23.6, 26.4.  A step on tiles
+// near which the two cross.  us per step, march against tiles: 640^2 FP64 34.5,
+// 28.9; 770^2 42.4, 37.9; 831^2 42.3, 43.4; 850^2 42.2, 43.6; 1000 x 610 41.9, 38.7;
+// 770^2 FP32 26.4, 24.7; 800^2 27.4, 27.5; 770^2 fp32_native 23.0, 21.0; 800^2 23.2,
+// 24.1.  (Either may be 10% the quicker near the line, as whole rounds of tiles
+// and of segments fall: 610 x 727 FP64 31.4, 37.3; 1200 x 520 mixed 25.6, 21.5.)
+// Nor more than 100 rows of strips per compute unit: a strip of few columns costs
+// a whole one in either kernel, and tall grids of them hold enough rows for the
+// march (4 x 50000 FP64 145, 189; 4 x 25000 86, 100, where the march's plan is the
+// worse one on most widths).  A step on tiles
 // takes about as long as the wavefronts on the busiest compute unit, ceil(tiles
 // / compute units) (R + 2), and longer by the root of the residency lost where
 // they come in several rounds of tiles of R + 2 wavefronts that do not fill it
-// (512^2 FP64: 10 rows 20.2, 6 rows 23.7; 900^2: 6 rows 50.2, 14 rows 53.1).
+// (512^2 FP64: 10 rows 21.0, 6 rows 23.7; 927^2: 6 rows 50.2, 14 rows 53.1).
 // The rows with the least of that are taken, among equals the fewest.
 // E2D_TILE_ROWS gives the rows (0: march), and any E2D_FUSED_* plan selects the
 // march it describes.
@@ -870,6 +876,7 @@ static int plan_tile_rows(const Grid& g, int waves_per_cu, int most_cells) {
                            "E2D_FUSED_CHUNK", "E2D_FUSED_TILE", "E2D_FUSED_PACK"})
     if (getenv(name)) return 0;
   const int64_t strips = (g.nx + kStripOut - 1) / kStripOut;
+  if (strips * g.ny > 100 * static_cast<int64_t>(cus)) return 0;
   int best = 0;
   double least = 0.0;
   for (int rows = 1; rows <= kTileMaxRows; ++rows) {
