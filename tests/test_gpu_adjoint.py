@@ -622,7 +622,7 @@ def test_marching_adjoint_equals_separate_passes(gpu_lib, prec, monkeypatch):
 
 
 # a single strip and two (58 columns each), tiles higher than the grid, rows that do not divide
-@pytest.mark.parametrize("rows", [1, 2, 7, 10])
+@pytest.mark.parametrize("rows", [1, 2, 6, 7, 10])
 @pytest.mark.parametrize("nx, ny, bc, st", [(4, 4, (1, 1, 1, 1), 1), (54, 9, (1, 2, 3, 1), 2), (57, 31, (3, 3, 2, 1), 1),
                                             (121, 23, (2, 1, 3, 3), 0)])
 def test_adjoint_tiles_equal_the_march(gpu_lib, monkeypatch, nx, ny, bc, st, rows):

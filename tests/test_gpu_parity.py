@@ -37,6 +37,18 @@ def _params(nx, ny=None, impl=0, prec=e2d.PREC_FP64, **kw):
     return p
 
 
+# implementation versions with the kernel of version 0 on small grids: tiles, the default
+# there, and the march (E2D_TILE_ROWS=0), the default on large ones
+IMPLS = [(0, None), (0, "0"), (1, None), (2, None)]
+
+
+def _tile_rows(monkeypatch, rows):
+    if rows is None:
+        monkeypatch.delenv("E2D_TILE_ROWS", raising=False)
+    else:
+        monkeypatch.setenv("E2D_TILE_ROWS", rows)
+
+
 # ---------------------------------------------------------------------------
 # pointwise device numerics vs the reference's routines
 
@@ -70,9 +82,10 @@ RUNS = ["diag128_fp64", "implode128_fp64", "diag128_fp32", "implode64_fp32_mc",
         "implode50x30_fp64_mixedbc"]
 
 
-@pytest.mark.parametrize("impl", [0, 1, 2])
+@pytest.mark.parametrize("impl, tile", IMPLS)
 @pytest.mark.parametrize("name", RUNS)
-def test_run_fixture_host_loop(gpu_lib, golden, name, impl):
+def test_run_fixture_host_loop(gpu_lib, golden, monkeypatch, name, impl, tile):
+    _tile_rows(monkeypatch, tile)
     d, nx, ny, steps, ic, prec, kw = _fixture_case(golden, name)
     with e2d.HydroRun(_params(nx, ny, impl, prec, **kw)) as run:
         run.init(ic)
@@ -83,10 +96,11 @@ def test_run_fixture_host_loop(gpu_lib, golden, name, impl):
     assert _same(u2, d["u2_end"]), _diff_report(u2, d["u2_end"])
 
 
-@pytest.mark.parametrize("impl", [0, 1, 2])
+@pytest.mark.parametrize("impl, tile", IMPLS)
 @pytest.mark.parametrize("name", ["diag128_fp64", "diag128_fp32", "implode40x48_fp64_periodic"])
-def test_run_fixture_device_loop(gpu_lib, golden, name, impl):
+def test_run_fixture_device_loop(gpu_lib, golden, monkeypatch, name, impl, tile):
     """e2d_run_steps keeps dt on the device; results equal the host loop's."""
+    _tile_rows(monkeypatch, tile)
     d, nx, ny, steps, ic, prec, kw = _fixture_case(golden, name)
     with e2d.HydroRun(_params(nx, ny, impl, prec, **kw)) as run:
         run.init(ic)
@@ -138,9 +152,10 @@ SIZES = [(4, 4, (1, 1, 1, 1)), (61, 17, (1, 2, 3, 1)), (121, 33, (3, 3, 3, 3)),
          (60, 16, (2, 2, 2, 2)), (7, 130, (1, 3, 2, 1)), (80, 23, (3, 3, 2, 1)), (80, 41, (2, 1, 3, 3))]
 
 
-@pytest.mark.parametrize("impl", [0, 1, 2])
+@pytest.mark.parametrize("impl, tile", IMPLS)
 @pytest.mark.parametrize("nx,ny,bc", SIZES)
-def test_sizes_vs_oracle(gpu_lib, nx, ny, bc, impl):
+def test_sizes_vs_oracle(gpu_lib, monkeypatch, nx, ny, bc, impl, tile):
+    _tile_rows(monkeypatch, tile)
     steps = 25
     kw = dict(boundary_type_xmin=bc[0], boundary_type_xmax=bc[1], boundary_type_ymin=bc[2],
               boundary_type_ymax=bc[3], slope_type=2)
@@ -156,7 +171,7 @@ def test_sizes_vs_oracle(gpu_lib, nx, ny, bc, impl):
     assert _same(u2, o.get(U2)), _diff_report(u2, o.get(U2))
 
 
-# segment plans of the fused step: long rows, short rows, percent of rows in
+# segment plans of the march: long rows, short rows, percent of rows in
 # long segments, strips per tile of the segment numbering (E2D_FUSED_SEG_ROWS /
 # _SHORT_ROWS / _LONG_PCT / _TILE); None = default.  At 130 columns there are
 # 3 strips: tile 2 leaves a last tile of one strip, 4 is clamped to 3.
@@ -164,7 +179,7 @@ def test_sizes_vs_oracle(gpu_lib, nx, ny, bc, impl):
 # at 130 columns the last strip has 10 output columns and is packed unless PACK is 0
 PLANS = [(None, None, None, None, None), (5, 2, 60, None, None), (3, 1, 0, None, None), (7, 3, 100, None, None),
          (1, 1, 75, None, None), (40, 7, 90, None, None), (None, None, None, 2, None), (None, None, None, 3, None),
-         (5, 2, 60, 4, None), (None, None, None, None, 0), (5, 2, 60, None, 0)]
+         (5, 2, 60, 4, None), (None, None, None, None, 0), (5, 2, 60, None, 0), "tiles"]
 
 
 @pytest.mark.parametrize("plan", PLANS)
@@ -172,9 +187,11 @@ PLANS = [(None, None, None, None, None), (5, 2, 60, None, None), (3, 1, 0, None,
 def test_segment_plans_vs_oracle(gpu_lib, monkeypatch, plan, prec, kind):
     """Whatever the split of each strip's rows into long and short segments,
     and however they are spread over the XCDs, the fused step gives the
-    oracle's bits (device-resident dt loop, 20 steps, 130 x 151)."""
+    oracle's bits (device-resident dt loop, 20 steps, 130 x 151); so does the
+    step on tiles, which a grid of that size takes by itself."""
+    _tile_rows(monkeypatch, None if plan == "tiles" else "0")
     for name, v in zip(("E2D_FUSED_SEG_ROWS", "E2D_FUSED_SHORT_ROWS", "E2D_FUSED_LONG_PCT", "E2D_FUSED_TILE",
-                        "E2D_FUSED_PACK"), plan):
+                        "E2D_FUSED_PACK"), [None] * 5 if plan == "tiles" else plan):
         if v is None:
             monkeypatch.delenv(name, raising=False)
         else:
@@ -194,16 +211,38 @@ def test_segment_plans_vs_oracle(gpu_lib, monkeypatch, plan, prec, kind):
     assert _same(u2, o.get(U2)), _diff_report(u2, o.get(U2))
 
 
+# FP64 grids whose segments are all of one length (4 to 9 rows a wavefront, all of them resident):
+# 850 columns leave a packed last strip (10 columns in version 0, 14 of 56 in version 2), 1030 one
+# in version 0 only, 1000 and 1300 none; the last segment of a strip may be shorter
+@pytest.mark.parametrize("impl, nx, ny", [(0, 850, 850), (0, 1030, 900), (0, 1000, 911), (0, 1300, 1200),
+                                          (2, 850, 760), (2, 1030, 900)])
+def test_one_length_segments_vs_oracle(gpu_lib, impl, nx, ny):
+    steps = 4
+    o = Oracle(nx, ny, bc=(1, 2, 3, 3))
+    o.init(IC_DIAG)
+    o.run(steps)
+    o.compute_dt(steps % 2)
+    with e2d.HydroRun(_params(nx, ny, impl, boundary_type_xmax=2, boundary_type_ymin=3, boundary_type_ymax=3)) as run:
+        run.init("diag")
+        run.make_boundaries(0)
+        run.run_steps(steps)
+        u, u2 = run.download(0), run.download(1)
+        assert run.invdt == o.invdt
+    assert _same(u, o.get(U)), _diff_report(u, o.get(U))
+    assert _same(u2, o.get(U2)), _diff_report(u2, o.get(U2))
+
+
 @pytest.mark.parametrize("prec", [e2d.PREC_FP32_NATIVE, e2d.PREC_MIXED])
 @pytest.mark.parametrize("nx, ny", [(130, 151), (80, 64)])
 def test_native_variants_independent_of_the_plan(gpu_lib, monkeypatch, prec, nx, ny):
     """fp32_native and mixed have no oracle of their own; their bits must not
-    depend on how the fused step splits the grid: the default plan (last strip
-    packed in 16- or 32-lane groups), the unpacked plan and a percentage plan
-    with short segments give the same state after 20 steps."""
+    depend on how the fused step splits the grid: tiles, the march's default plan
+    (last strip packed in 16- or 32-lane groups), its unpacked plan and a
+    percentage plan with short segments give the same state after 20 steps."""
     out = []
-    for env in ({}, {"E2D_FUSED_PACK": "0"}, {"E2D_FUSED_SEG_ROWS": "3", "E2D_FUSED_LONG_PCT": "50"}):
-        for name in ("E2D_FUSED_PACK", "E2D_FUSED_SEG_ROWS", "E2D_FUSED_LONG_PCT"):
+    for env in ({}, {"E2D_TILE_ROWS": "0"}, {"E2D_FUSED_PACK": "0"},
+                {"E2D_FUSED_SEG_ROWS": "3", "E2D_FUSED_LONG_PCT": "50"}):
+        for name in ("E2D_TILE_ROWS", "E2D_FUSED_PACK", "E2D_FUSED_SEG_ROWS", "E2D_FUSED_LONG_PCT"):
             monkeypatch.delenv(name, raising=False)
         for name, v in env.items():
             monkeypatch.setenv(name, v)
