@@ -69,7 +69,6 @@ struct DualMath {
   static E2D_HDI Dual div_inv(Dual a, Dual b, Dual) { return div(a, b); }
   static E2D_HDI Dual recip(Dual) { return Dual(0.0, 0.0); }
   static E2D_HDI Dual recip_near(Dual, Dual) { return Dual(0.0, 0.0); }
-  static E2D_HDI Dual inv_given(Dual b, Dual) { return div(Dual(1.0, 0.0), b); }
   static E2D_HDI bool quot_gt(Dual a, Dual d, Dual tol, Dual h) { return Base::quot_gt(a.v, d.v, tol.v, h.v); }
 };
 

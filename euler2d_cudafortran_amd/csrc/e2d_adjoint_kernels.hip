@@ -5,7 +5,8 @@
 //
 // Five deterministic passes (every output element is written by one thread,
 // which gathers its contributions in a fixed order):
-//   1. k_adj_prim   q = prim(u) on all cells (input buffer boundary-filled first)
+//   1. k_adj_prim   q = prim(u) on all cells (input buffer boundary-filled first;
+//                   k_adj_tile, below, forms the ghost cells as it loads them)
 //   2. k_adj_faces  per face: flux bar from lam, Riemann adjoint -> bars of the
 //                   two face states (stored in the XMIN/XMAX/YMIN/YMAX slot of
 //                   the cell that owns each state)
@@ -651,7 +652,7 @@ __device__ __forceinline__ void adj_march_gather_body(const AdjArgs<P>& a) {
   const T pb = prim_at(a, cl, row(ra - 1), qb);
   // bits 0, 1, 2: row r+1, r, r-1 holds a cell that takes the limiter's long form
   unsigned long_rows = (any_long_slope(pa) ? 2 : 0) + (any_long_slope(pb) ? 1 : 0);
-  // row r-1, carried: slopes, trace sources and the bars of its xmin, xmax, ymin face states
+  // row r-1, carried: slopes and trace sources
   T pdx[4], pdy[4], ps[4];
   // carried in LDS: partial sum of the last completed row, its plus part, the
   // primitives of row r-2, and row r-1's face bars
@@ -892,10 +893,10 @@ __global__ __launch_bounds__(64 * kAdjWaves) __attribute__((amdgpu_waves_per_eu(
 // another tile forms and go to the seam buffer, as there.  The input's ghost
 // cells are formed on load and written back (no fill before this kernel).
 // The values and their order are k_adj_march_gather's, so the bits are the same.
-// us per adjoint step against the march, all kernels: 64^2 FP64 72.1, 30.0;
-// 256^2 84.1, 36.1; 512^2 81.8, 72.6; 512^2 FP32 65.2, 50.1 (a grid that small
-// gives the march one wavefront per SIMD or fewer, each with a chain of 6 or
-// more row iterations).
+// us per adjoint step, march against tiles, all kernels, the diagonal problem
+// after 100 steps: 64^2 FP64 51.4, 25.9; 256^2 58.7, 31.1; 512^2 63.9, 60.4; 512^2
+// FP32 53.7, 42.8 (a grid that small gives the march one wavefront per SIMD or
+// fewer, each with a chain of 6 or more row iterations).
 constexpr int kAdjTileMaxRows = 10;
 // resident wavefronts per SIMD: FP64 takes 155 VGPRs, the float variants 86-88
 template <class T>
@@ -1323,16 +1324,18 @@ __global__ __launch_bounds__(256) void k_adj_fold_frame(const AdjArgs<P> a) {
 }
 
 // Kernel sequence of an adjoint step, all giving the same bits:
+//   tiles   k_adj_tile + k_adj_seam, on grids that plan_adjoint_tile names
 //   fused   k_adj_march_gather + k_adj_seam
 //   march   k_adj_march + k_adj_gather_march (bars of q and of the slopes
 //           through HBM)
 //   separate  k_adj_prim, k_adj_faces, k_adj_cells, k_adj_gather (face bars
 //           through HBM as well)
+// k_adj_fold_frame follows each, and k_boundaries goes before all but the tiles.
 // E2D_ADJOINT_PASSES=fused|march|separate chooses; fused is the default
-// (2048^2, dense lam: FP64 778 us fused, 796 us march; FP32 477 us fused,
-// 527 us march).  The fused kernel writes lam_out while other wavefronts still
-// read lam_in, so an aliased call (lam_out == lam_in) runs march, whose gather
-// reads and writes each element of lam in the same thread.
+// (2048^2, dense lam, us: FP64 437 fused, 601 march, 1144 separate; FP32 270,
+// 365, 660).  The fused kernel and the tiles write lam_out while other wavefronts
+// still read lam_in, so an aliased call (lam_out == lam_in) runs march, whose
+// gather reads and writes each element of lam in the same thread.
 enum class Passes { kFused, kMarch, kSeparate };
 Passes adjoint_passes(bool aliased) {
   Passes p = Passes::kFused;
@@ -1349,7 +1352,7 @@ Passes adjoint_passes(bool aliased) {
 // rows/340, clamped to [4, 16].  The kernel holds 2 wavefronts per SIMD, so
 // short segments (many wavefronts, several rounds) balance the data-dependent
 // Riemann work best: measured at 2048^2 FP64 with a dense lam, 4-7 rows give
-// 860-880 us per adjoint step, 12 rows 896 us, 18 rows 950 us, 24 rows 1030 us.
+// 605-622 us per adjoint step, 12 rows 629 us, 18 rows 655 us, 24 rows 659 us.
 int march_seg_rows(int rows) {
   if (const char* env = getenv("E2D_ADJOINT_SEG_ROWS")) {
     const int r = atoi(env);
@@ -1368,13 +1371,13 @@ static int adj_env(const char* name, int dflt) {
 // rows: long segments of about rows/170 rows (within [4, 16];
 // E2D_ADJOINT_SEG_ROWS overrides) over the lower 75% of the rows
 // (E2D_ADJOINT_LONG_PCT), short ones of a third of that
-// (E2D_ADJOINT_SHORT_ROWS; 4 rows against 3: FP64 720 -> 715 us, FP32
-// 441 -> 430 us, mixed 386 -> 380 us) over the rest, dealt to the XCDs in chunks of 16
+// (E2D_ADJOINT_SHORT_ROWS; 4 rows against 3: FP64 441 -> 436 us, FP32
+// 272 -> 270 us, mixed 253 -> 250 us) over the rest, dealt to the XCDs in chunks of 16
 // segments (E2D_ADJOINT_CHUNK), so every XCD ends on short segments.
 // Measured at 2048^2 with a dense lam, us per adjoint step against uniform
-// 6-row segments: FP64 765 -> 721, FP32 481 -> 437, mixed 417 -> 384; 16-row
-// long segments suit FP64 (715) but not the float kernels, which hold 3
-// wavefronts per SIMD (518 and 440).  Returns the number of blocks.
+// 6-row segments: FP64 477 -> 437, FP32 296 -> 270, mixed 276 -> 250; 16-row
+// long segments suit FP64 (430) but not the float kernels, which hold 3
+// wavefronts per SIMD (284 and 262).  Returns the number of blocks.
 template <class P>
 int plan_adjoint_segments(AdjArgs<P>& a, int nstrips, int rows) {
   int R = adj_env("E2D_ADJOINT_SEG_ROWS", 0);
@@ -1411,13 +1414,16 @@ int gather_seg_rows() {
 
 // Rows per tile of k_adj_tile, or 0 for the march.  Tiles up to 1,500 cells per
 // compute unit in FP64 (about 620^2) and 4,100 in the float variants (1024^2),
-// where the two cross (march against tiles, us per adjoint step with the seam
-// and frame kernels: 512^2 FP64 72.5, 67.0, 600^2 94.8, 84.5, 300 x 1200 89.1,
-// 95.6; 900^2 FP32 93.3, 92.7, 1024^2 112.8, 112.2, mixed 102.9, 101.5).  2 rows, whose 4
+// near which the two cross (march against tiles, us per adjoint step of the bumps'
+// first state with the seam and frame kernels: 512^2 FP64 71.9, 67.5, 600^2 94.6,
+// 79.8, 1200 x 300 91.2, 79.3, 300 x 1200 88.9, 90.9; 512^2 FP32 63.4, 46.9, 1024^2
+// 111.9, 109.7, mixed 101.3, 100.1; 900^2, on the slower side as its tiles fall, FP32
+// 85.3, 91.7).  Nor more than 100 rows of strips per compute unit, as for the step
+// (4 x 50000 FP64 429, 650).  2 rows, whose 4
 // wavefronts spread over the SIMDs, while one round of such tiles holds the
-// grid (128^2 FP64 25.3 us, with 7 rows 40.6); beyond, 7 rows in FP64 and 6 in
-// the float variants, which form less twice (512^2: 72.6 against 80.3 with 2
-// rows; FP32 50.1 against 51.2).  E2D_ADJOINT_TILE_ROWS gives the rows (0: march);
+// grid (128^2 FP64 24.4 us, with 7 rows 33.6); beyond, 7 rows in FP64 and 6 in
+// the float variants, which form less twice (512^2: 60.4 against 68.8 with 2
+// rows; FP32 42.8 against 44.1).  E2D_ADJOINT_TILE_ROWS gives the rows (0: march);
 // E2D_ADJOINT_PASSES=fused or a segment plan of the march selects the march.
 int plan_adjoint_tile(const Grid& g, size_t elem) {
   const int forced = adj_env("E2D_ADJOINT_TILE_ROWS", -1);

@@ -65,7 +65,8 @@ int validate(const e2d_params* p) {
   // The Riemann solver's radicands are bounded below by gamma0 smallr^2 smallp
   // (1 - gamma6) (densities and pressures are floored at smallr and
   // rho smallp, and p* >= 0); the step takes their square roots without a
-  // zero case, so that bound must be a positive normal double.
+  // zero case, so that bound must be a positive normal double (in binary32 it
+  // may be less: such FP32 runs take the roots of low_floors).
   const double smallp = p->smallc * p->smallc / p->gamma0;
   const double gamma6 = (p->gamma0 + 1.0) / (2.0 * p->gamma0);
   const double radicand_floor = p->gamma0 * p->smallr * (p->smallr * smallp) * (1.0 - gamma6);

@@ -12,9 +12,10 @@ namespace e2d {
 
 // Host-side trace range (roctx; rocprofv3 --marker-trace records it), named
 // after the reference's NVTX ranges (serial_ref/m_run.f90:195,264,336,387,502,571:
-// godunov_compute, compute_dt, computeAndStoreFluxes, make_boundaries; the
-// conversion and the update have no kernels of their own).  It spans the
-// enqueue of the kernels, which the trace attributes to it.
+// godunov_compute, compute_dt, convertToPrimitives, computeAndStoreFluxes,
+// updateHydro, make_boundaries).  It spans the enqueue of the kernels, which the
+// trace attributes to it; the conversion, the fluxes and the update of versions
+// 1 and 2 are one kernel, and their ranges lie around it, each the whole launch.
 struct TraceRange {
   explicit TraceRange(const char* name) { roctxRangePushA(name); }
   ~TraceRange() { roctxRangePop(); }

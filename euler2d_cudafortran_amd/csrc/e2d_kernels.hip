@@ -38,11 +38,12 @@ namespace e2d {
 // s kOut + kFirst - kHalo + l, and the strip's own columns are those of the
 // lanes kHalo .. 63 - kHalo.  The fused step: 60 columns from the first
 // interior one, 2 halo columns each side.  With stages (STAGES != 0): 56
-// columns from column 0, so that every row that is stored begins and ends on a
-// 64-byte boundary.  With partial 64-byte pieces at every strip's edge, and
-// with stores that the caches keep, the stage arrays wrote at 3 TB/s; aligned
-// and non-temporal, at 5 (version 1 in FP64 at 2048^2, per step: 570 us,
-// aligned 530, both 385).
+// columns from column 0, so that every row of 8-byte values that is stored
+// begins and ends on a 64-byte boundary (of 4-byte ones, 224 bytes, every second
+// strip's begins within a piece).  With partial 64-byte pieces at every strip's
+// edge, and with stores that the caches keep, the stage arrays wrote at 3 TB/s;
+// aligned and non-temporal, at 5 (version 1 in FP64 at 2048^2, per step: 570 us,
+// aligned 530, both 385; now, with 2 wavefronts per SIMD, 340, in FP32 285).
 template <int STAGES>
 struct Strip {
   static constexpr int kHalo = STAGES ? 4 : 2, kOut = 64 - 2 * kHalo, kFirst = STAGES ? 0 : 2;
@@ -550,8 +551,8 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) __attribute__((amdgpu_waves_pe
 // same routines on the same operands, so the bits are the same.
 // Each wavefront holds one row only: 80 VGPRs in FP64 (6 wavefronts per SIMD,
 // against the march's 3) and about 50 in the float variants.  us per FP64 step,
-// march against tiles: 128^2 11.1, 8.1; 250 x 130 11.3, 8.4; 512^2 21.4, 20.2;
-// 768^2 44.8, 37.3.  On grids that fill the device (2048^2: 178 against 225)
+// march against tiles: 128^2 11.4, 8.4; 250 x 130 11.5, 8.7; 512^2 22.9, 20.5;
+// 768^2 40.9, 36.4.  On grids that fill the device (2048^2: 157 against 208)
 // the barriers and the rows formed twice cost more than the chain saves.
 constexpr int kTileMaxRows = 14;
 template <class P>
@@ -763,9 +764,9 @@ static int waves_per_simd(const void* kernel) {
 // (which leaves 9% of the long segments for a second round); FP32 12 rows
 // 134-136 against 139-140; fp32_native 106.3 against 107.1; 4096^2 FP64 37 rows
 // (two rounds) 711 against 716, 74 rows (one round) 719.  Where the rounds
-// would give segments of fewer than 8 rows (grids up to about 1200^2) the
-// plan is segments of one length in FP64 (below), and long segments of
-// fused_seg_rows rows over 75% of the rows otherwise.
+// would give segments of fewer than 8 rows (grids up to about 1300^2 in FP64,
+// 1600^2 in FP32) the plan is segments of one length in FP64 (below), and long
+// segments of fused_seg_rows rows over 75% of the rows otherwise.
 // E2D_FUSED_SEG_ROWS or E2D_FUSED_LONG_PCT select that plan with the given
 // values, E2D_FUSED_SHORT_ROWS the short length; the environment is read at
 // every launch.  Returns the number of blocks.
@@ -809,10 +810,13 @@ static int plan_segments(StepArgs<P>& a, int ncols, int ny, int wps, int residen
       npk = pk;
     }
   }
-  // FP64 grids of about 800^2 to 1400^2: segments of one length, the least that
-  // lets all of them start at once.  us per step against long segments over 75%
-  // of the rows: 850^2 44.1 against 52.8, 1024^2 57.7 against 66.4, 1200^2 73.3
-  // against 82.7, 1400^2 93.4 against 93.9 (the float variants gain and lose 2%).
+  // FP64 grids of about 700^2 (version 0 marches from 830^2) to 1300^2: segments
+  // of one length, the least that lets all of them start at once.  us per step
+  // against long segments over 75% of the rows: 850^2 42.2 against 50.8, 1024^2
+  // 56.2 against 64.4, 1200^2 70.7 against 78.1, 1300^2 82.5 against 87.1 (the float
+  // variants gain and lose 2%).  They lose where the other plan's wavefronts all
+  // start at once too, on tall grids of about ten strips: 611 x 1294 49.5 against
+  // 46.0, 629 x 2240 77.3 against 69.2.
   if (R == 0 && !forced && sizeof(typename P::T) == 8) {
     int rows = 1;
     auto wavefronts = [&](int r) {

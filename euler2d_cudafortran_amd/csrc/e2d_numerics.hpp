@@ -110,16 +110,20 @@ struct FastMath {
 // nonzero operands whose binary exponents stay far from the double limits
 // (|log2| below ~700; the solver's values span about 1e-22..1e9).  These are
 // the Newton-Raphson (division) and Goldschmidt (square root) cores of the
-// IEEE sequences the compiler emits for a / b and sqrt(x) on gfx950, without
+// IEEE sequences the compiler emits for a / b and sqrt(x) on gfx950 (with
+// another reciprocal, below), without
 // the range scaling (v_div_scale, ldexp by 2^256) and special-value fixup
 // (v_div_fixup, class tests) that act only outside that range.  Inside it the
-// results are the IEEE results bit for bit, except that a zero quotient is +0
+// results are the IEEE results bit for bit (roots; quotients on the samples below
+// and the hard cases of the tests), except that a zero quotient is +0
 // whatever the sign of the numerator; a zero radicand returns zero (sqrt; the
 // core alone, sqrt_pos, returns NaN for it and is the IEEE result for every
-// positive radicand in the range).
+// positive radicand in the range; an infinite one returns NaN).
 //
-// The FP32 overloads do the same for binary32 (exponents within about +-90,
-// the solver's 1e-22..1e9 again).  The reciprocal seed (v_rcp_f32, within 1 ulp)
+// The FP32 overloads do the same for binary32: radicands from 2^-102, where
+// x - g g is still exact, and dividends from about 2^-102 (below, the remainder's
+// own rounding shows in the last bit of the quotient); LowFloorMath is for runs
+// whose floors allow smaller radicands.  The reciprocal seed (v_rcp_f32, within 1 ulp)
 // after one Newton step is the correctly rounded reciprocal for every one of
 // the 2^23 mantissas, and one remainder correction of a r gives the correctly
 // rounded quotient for every one of the 2^46 pairs of mantissas (both checked
@@ -176,7 +180,8 @@ struct RangedMath {
   // e = 1 - b r: the error left is e^3 (2^-73) and the last rounding, as after
   // the two Newton steps of the IEEE sequence (2^-97), in three fmas instead of
   // four.  Of 2^30 random divisors 11 reciprocals differ from the two-step one
-  // by an ulp, and none of as many quotients.
+  // by an ulp, and none of as many quotients: that every quotient is the same is
+  // sampled, not proven.
   static __device__ __forceinline__ double recip(double b) {
     const double r = __builtin_amdgcn_rcp(b);
     const double e = __builtin_fma(-b, r, 1.0);
